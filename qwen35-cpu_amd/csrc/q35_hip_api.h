@@ -102,6 +102,8 @@ __device__ __forceinline__ void q35_materialize(float &x) { asm volatile("" : "+
 // A wave-uniform value moved into a scalar register (every lane holds the
 // same value; the compiler then treats what derives from it as uniform).
 __device__ __forceinline__ int q35_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// Bit l of the result: whether lane l's predicate holds (all 64 lanes call it).
+__device__ __forceinline__ unsigned long long q35_ballot(bool p) { return __ballot(p); }
 // Raw (stride 0) buffer resource over [base, base + extent) with a
 // wave-uniform base: a load takes a per-lane byte offset and a wave-uniform
 // one (a scalar register, so per-iteration offsets cost no VALU work); an

@@ -384,6 +384,16 @@ inline int q35emu_sdot4(uint32_t a, uint32_t b, int c) {
   return c;
 }
 #define Q35_SDOT4(a, b, c) q35emu_sdot4(static_cast<uint32_t>(a), static_cast<uint32_t>(b), (c))
+inline unsigned long long q35_ballot(bool p) {
+  auto &ctx = ::q35emu::t_ctx;
+  auto &slots = ctx.launch->slots_a[ctx.wave];
+  slots[ctx.lane] = p ? 1u : 0u;
+  ::q35emu::wave_sync();
+  unsigned long long m = 0;
+  for (int l = 0; l < 64; ++l) m |= static_cast<unsigned long long>(slots[l]) << l;
+  ::q35emu::wave_sync();
+  return m;
+}
 inline void lds_barrier() { __syncthreads(); }
 inline void wave_lds_sync() { ::q35emu::wave_sync(); }
 inline void q35_compiler_fence() { asm volatile("" ::: "memory"); }

@@ -1,5 +1,5 @@
 """Operator forms at the sizes where their launches change shape: run and
-vector edges of the convolution.
+vector edges of the convolution, candidate lists with ties and few tokens.
 Each against the oracle's token-by-token or single-value form, within the
 rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
@@ -38,3 +38,34 @@ def test_conv1d_runs(q, ctx, orc, batch, ch, kern, begin, end, extra, in_place):
         if hist:
             want_state[(ring + p) % hist, begin:end] = x[p, begin:end]
     np.testing.assert_array_equal(dstate.download(), want_state)
+
+
+@pytest.mark.parametrize("vocab,k", [(64, 64), (264, 1), (264, 64), (8192, 20), (8192, 64)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_candidates_against_sort(q, ctx, vocab, k, ties):
+    """The candidate list equals a descending sort of the raw logits (lower
+    token first among equals): few tokens per slice, all logits equal (a zero
+    hidden row), penalized tokens, k up to 64."""
+    from tests.model_util import build_small_model, small_dims, upload_model
+    d, sched = small_dims()
+    d["vocab"] = vocab
+    model = upload_model(q, ctx, d, sched, build_small_model(d, sched, seed=vocab))
+    rt = q.Runtime(model, max_slots=1, max_batch=1, max_context=64, page_tokens=16, use_graphs=False)
+    prompt = np.arange(0, vocab, 3, dtype=np.int32)[:40]
+    slot = rt.slot_alloc(prompt)
+    rng = np.random.default_rng(k)
+    hidden = np.zeros(d["hidden"], np.float32) if ties else rng.standard_normal(d["hidden"]).astype(np.float32)
+    print(f"candidates vocab {vocab} k {k} ties {ties}", flush=True)
+    cand, raw = rt.head_candidates(slot, hidden, k, 1.25, penalty=1.3, raw_logits=True)
+    v = raw.copy()
+    hit = rt.slot_counts(slot) > 0
+    v[hit] = np.where(v[hit] > 0, v[hit] / np.float32(1.3), v[hit] * np.float32(1.3))
+    v = (v * np.float32(1.25)).astype(np.float32)
+    # the kernel's order puts +0 above -0
+    key = np.where(v == 0, np.where(np.signbit(v), -1e-45, 0.0), v.astype(np.float64))
+    order = np.lexsort((np.arange(vocab), -key))[:k]
+    np.testing.assert_array_equal(cand["token"][:k], order)
+    np.testing.assert_array_equal(cand["value"][:k].view(np.uint32), v[order].view(np.uint32))
+    assert np.all(cand["token"][k:] == -1) and np.all(np.isneginf(cand["value"][k:]))
+    rt.close()
+    model.close()
