@@ -290,6 +290,14 @@ int dot4_matmul_run(Context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_blo
     if (e != hipSuccess) return hip_error(ctx, e, "dot4 GEMV kernel");
     return Q35_OK;
   }
+  if (out != nullptr && dots == nullptr && index == nullptr && !exact &&
+      gemm_direct_fits(static_cast<int>(rows), nb, vectors, ctx->cu_count)) {
+    const hipError_t e = launch_gemm_direct(m, x4 != nullptr ? static_cast<const void *>(x4) : x1, x4 != nullptr,
+                                            static_cast<int>(rows), nb, static_cast<int>(vectors), out,
+                                            static_cast<long long>(stride), ctx->cu_count, ctx->stream);
+    if (e != hipSuccess) return hip_error(ctx, e, "direct DOT4 GEMM kernel");
+    return Q35_OK;
+  }
   const size_t tiles = (chunk + 15) / 16;
   const size_t code_bytes = align256(tiles * 64 * static_cast<size_t>(nb) * sizeof(uint64_t));
   const size_t scale_bytes = align256(tiles * 16 * static_cast<size_t>(nb) * sizeof(float));
@@ -375,8 +383,11 @@ int matmul_entry(q35_context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_bl
                      vectors > static_cast<size_t>(kMaxTokens);
   const size_t chunk = dense ? std::min<size_t>((vectors + 15) / 16 * 16, kDenseChunk) : kMaxTokens;
   void *scratch = nullptr;
-  // one to four plain outputs: the single-launch GEMV, no scratch
-  if (out != nullptr && dots == nullptr && index == nullptr && !exact && vectors <= kMatvecMaxVectors)
+  // plain outputs of one to four vectors (the GEMV) or of a batch that the
+  // direct GEMM takes: one launch, no scratch
+  if (out != nullptr && dots == nullptr && index == nullptr && !exact &&
+      (vectors <= static_cast<size_t>(kMatvecMaxVectors) ||
+       gemm_direct_fits(static_cast<int>(rows), static_cast<int>(blocks), vectors, ctx->cu_count)))
     return dot4_matmul_run(ctx, m, x4, x1, out, dots, rows, vectors, blocks, stride, exact, index, value, counts,
                            penalties, nullptr, chunk);
   st = scratch_get(ctx,

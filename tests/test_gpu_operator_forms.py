@@ -1,5 +1,6 @@
 """Operator forms at the sizes where their launches change shape: run and
-vector edges of the convolution, candidate lists with ties and few tokens.
+vector edges of the convolution, candidate lists with ties and few tokens,
+batches of the direct GEMM.
 Each against the oracle's token-by-token or single-value form, within the
 rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
@@ -69,3 +70,53 @@ def test_candidates_against_sort(q, ctx, vocab, k, ties):
     assert np.all(cand["token"][k:] == -1) and np.all(np.isneginf(cand["value"][k:]))
     rt.close()
     model.close()
+
+
+@pytest.mark.parametrize("rows,blocks", [(8, 1), (8, 8), (24, 9), (40, 3), (72, 33), (136, 112), (16, 260)])
+@pytest.mark.parametrize("tokens", [5, 8, 15, 16, 17, 36, 64, 68])
+def test_direct_gemm_forms(q, ctx, orc, rows, blocks, tokens):
+    """X4 and X1 activations, row and token tails, one split to more than 16:
+    every output within the rounding of its chain of the float64 product, and
+    the same bits whatever the layout and the batch (the chain of an output
+    depends on rows and blocks only); rows past the stride's end untouched."""
+    rng = np.random.default_rng(rows * 1000 + blocks * 10 + tokens)
+    cols = 32 * blocks
+    dm = ctx.array(orc.dot4_pack(orc.random_q4_blocks(rng, rows, cols), rows, blocks))
+    codes = rng.integers(-127, 128, size=(tokens, blocks, 32)).astype(np.int8)
+    scales = rng.uniform(0.001, 0.02, size=(tokens, blocks)).astype(np.float32)
+
+    def x1_blocks(c, s):
+        b = np.zeros((len(c), blocks), np.dtype([("s", "<f4"), ("sum", "<i2"), ("q", "i1", 32), ("pad", "<i2")]))
+        b["s"], b["sum"], b["q"] = s, c.sum(-1), c
+        return b
+
+    def x4_blocks(c, s):
+        b = np.zeros((len(c) // 4, blocks), np.dtype([("s", "<f4", 4), ("sum", "<i2", 4), ("q", "i1", (4, 32))]))
+        b["s"] = s.reshape(-1, 4, blocks).transpose(0, 2, 1)
+        b["q"] = c.reshape(-1, 4, blocks, 32).transpose(0, 2, 1, 3)
+        b["sum"] = b["q"].sum(-1)
+        return b
+
+    def run(call, blk, n, stride):
+        out = ctx.array(np.full((n, stride), 7.0, np.float32))
+        call(ctx, dm, ctx.array(blk.view(np.uint8)), out, rows, n, blocks, stride)
+        got = out.download()
+        assert np.all(got[:, rows:] == 7.0)
+        return got[:, :rows]
+
+    print(f"direct GEMM {rows} rows {blocks} blocks {tokens} tokens", flush=True)
+    got = run(q.q4_dot4_matmul_x1, x1_blocks(codes, scales), tokens, rows + 3)
+    # terms dot * d * s per block: the kernels' exact integer dots, in float64
+    pad = (-tokens) % 4
+    c4, s4 = np.concatenate([codes, codes[:pad]]), np.concatenate([scales, scales[:pad]])
+    dots = ctx.array(shape=(tokens + pad, rows, blocks), dtype=np.int32)
+    q.q4_dot4_block_dots(ctx, dm, ctx.array(x4_blocks(c4, s4).view(np.uint8)), dots, rows, tokens + pad, blocks)
+    tiles = dm.download().view(np.uint8).reshape(rows // 8, blocks, 144)
+    d = np.ascontiguousarray(tiles[..., :16]).view(np.float16).reshape(rows // 8, blocks, 8).transpose(0, 2, 1)
+    terms = dots.download()[:tokens] * d.reshape(rows, blocks).astype(np.float64) * scales[:, None, :].astype(np.float64)
+    bound = (blocks + 2) * 2.0 ** -24 * 2 * np.abs(terms).sum(-1)  # a rounding per product and per addition
+    assert np.all(np.abs(got - terms.sum(-1)) <= bound)
+    x4 = run(q.q4_dot4_matmul, x4_blocks(c4, s4), tokens + pad, rows + 4)
+    np.testing.assert_array_equal(x4[:tokens].view(np.uint32), got.view(np.uint32))
+    few = run(q.q4_dot4_matmul_x1, x1_blocks(codes[:5], scales[:5]), 5, rows)
+    np.testing.assert_array_equal(few.view(np.uint32), got[:5].view(np.uint32))
