@@ -177,9 +177,18 @@ hipError_t launch_gemm_direct(const q35_q4_0_block_x8 *w, const void *act, bool 
   a.out = out;
   a.stride = stride;
   a.vec_out = stride % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  int nt = tokens <= 16 ? 1 : tokens <= 32 ? 2 : 4;
+  // token tiles per workgroup: as few as keep the launch within 14 wavefronts
+  // per compute unit, where a workgroup's own latency sets the time (1024 x
+  // 3584, 64 vectors: 5.4 us with one tile, 10.2 with four); beyond that more
+  // tiles share each weight load and unpack (18432 x 2560, 64 vectors: 44.0 us
+  // with one tile, 32.1 with four)
+  const int waves = std::min(a.splits, 16), groups = (rows + 15) / 16, cus = cu_count > 0 ? cu_count : 256;
+  int nt = 1;
+  while (nt < 4 && 16 * nt < tokens &&
+         static_cast<long long>(groups) * ((tokens + 16 * nt - 1) / (16 * nt)) * waves > 14LL * cus)
+    nt <<= 1;
   while (nt > 1 && direct_lds(a.splits, nt) > kDirectMaxLds) nt >>= 1;
-  const dim3 grid((rows + 15) / 16, (tokens + 16 * nt - 1) / (16 * nt)), block(64 * std::min(a.splits, 16));
+  const dim3 grid(groups, (tokens + 16 * nt - 1) / (16 * nt)), block(64 * waves);
   const size_t lds = direct_lds(a.splits, nt);
 #define Q35_DIRECT(NT, KS)                                                                             \
   if (x4)                                                                                              \
