@@ -3,6 +3,8 @@
 // the int8 block dots run on the VALU dot4 unit, and each output row is the
 // reference's single fma chain over the blocks in order, so the results are
 // bit-exact (no split-K, no reduce kernel).
+#include <algorithm>
+
 #include "q35_device.h"
 #include "q35_internal.h"
 
@@ -10,8 +12,7 @@ namespace q35 {
 
 namespace {
 constexpr int kMvThreads = 256;
-// blocks per chain pass: 4 wavefronts x 8 block lanes x 4 blocks per lane
-constexpr int kMvPass = 128;
+constexpr int kMvStep = 32;  // blocks per step of a workgroup: 4 wavefronts x 8
 
 struct MvArgs {
   const uint8_t *w;    // Q4_0BlockX8 tiles [rows / 8][nb]
@@ -22,85 +23,97 @@ struct MvArgs {
   long long stride;  // output row stride (floats) between vectors
 };
 
-// One workgroup per 8-row tile group. Lane (r, j) of wavefront w owns row r
-// of the group and blocks j + 8 (w + 4 i) of each 128-block pass: it loads the
-// row's four body words (columns 8t..8t+7 of each word t) and the row's
-// scale, and per vector forms
-//   dot = sum_k (u_k - 8) a_k   (sdot4 of the nibbles against the codes,
-//                               then -8 times the code sum, all in int32),
-//   scale = half(d_r) * s_a      (q4_dot4.cpp:52-54),
-// which land in LDS. The first 8 * count lanes then run the row chains
-// result = fma(float(dot), scale, result) block by block
-// (q4_dot4.cpp:43-56, restated by q35o_dot4_matvec).
-template <int NV, bool X4>
+// One workgroup per 8-row tile group, STEPS steps of kMvStep blocks per pass.
+// Lane (j, h, t) = (lane / 8, lane / 4 % 2, lane % 4) of wavefront w takes block
+// j + 8w of a step: 16 bytes of its tile (the words of rows 4h .. 4h+3, columns
+// 8t .. 8t+7), so a wavefront reads eight tiles whole, and the eight codes of
+// those columns. Per vector it forms its part of the four rows' dots
+//   sum_k (u_k - 8) a_k   (sdot4 of the nibbles against the codes, on top of
+//                         -8 times their sum, all in int32);
+// two exchanges over t leave lane (h, t) with the whole dot of row 4h + t. The
+// dot and scale = half(d_r) * s_a (q4_dot4.cpp:52-54) land in LDS, and the
+// first 8 * count lanes run the row chains
+// result = fma(float(dot), scale, result) block by block (q4_dot4.cpp:43-56,
+// restated by q35o_dot4_matvec) while the next pass's loads are in flight.
+// Bound by latency: one round trip, the dots and the chain. With each lane
+// loading one row's four words (4 bytes each) and all 32 codes, 18432 x 2560
+// took 13.6 us a call and four X4 vectors 21.3, this form 6.8 and 10.7.
+template <int NV, bool X4, int STEPS>
 __global__ __launch_bounds__(kMvThreads) void dot4_matvec_kernel(MvArgs a) {
-  __shared__ q35_f32x2 fs[NV][8][kMvPass + 1];  // +1: the chain lanes' reads hit distinct banks
+  constexpr int kPass = kMvStep * STEPS;
+  __shared__ q35_f32x2 fs[NV][8][kPass + 1];  // +1: the chain lanes' reads hit distinct banks
   const int g = blockIdx.x;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane & 7, j = lane >> 3;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int t = lane & 3, h = (lane >> 2) & 1, j = lane >> 3, r = 4 * h + t;
   const uint8_t *tiles = a.w + static_cast<size_t>(g) * a.nb * 144;
   float res = 0.0F;
-  for (int b0 = 0; b0 < a.nb; b0 += kMvPass) {
-    const int n = min(kMvPass, a.nb - b0);
-    // every load of the pass first (slots past the pass read its last block
-    // and are not stored), then the dots
-    uint32_t wq[4][4], c[4][NV][8];
-    float dw[4], sa[4][NV];
+  q35_u32x4 wq[STEPS];
+  uint16_t dh[STEPS];
+  uint32_t c[STEPS][NV][X4 ? 2 : 3];
+  float sa[STEPS][NV];
+  // every load of a pass (slots past it read its last block and are not stored)
+  auto load = [&](int b0) {
+    const int n = min(kPass, a.nb - b0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int b = b0 + min(j + 8 * (wave + 4 * i), n - 1);
+    for (int i = 0; i < STEPS; ++i) {
+      const int b = b0 + min(j + 8 * wave + kMvStep * i, n - 1);
       const uint8_t *tile = tiles + static_cast<size_t>(b) * 144;
-      const uint32_t *q = reinterpret_cast<const uint32_t *>(tile + 16 + 4 * r);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) wq[i][t] = Q35_LOAD_NT(q + 8 * t);
-      dw[i] = half_bits_to_float(reinterpret_cast<const uint16_t *>(tile)[r]);
+      wq[i] = Q35_LOAD_NT(reinterpret_cast<const q35_u32x4 *>(tile + 16 + 32 * t + 16 * h));
+      dh[i] = reinterpret_cast<const uint16_t *>(tile)[r];
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        if (X4) {
+        if constexpr (X4) {
           // scales[4], sums[4], qs[4][32]: vector v's codes at byte 24 + 32 v
           const uint8_t *blk = a.act + static_cast<size_t>(b) * 152;
           sa[i][v] = reinterpret_cast<const float *>(blk)[v];
-          const q35_u32x2 *cp = reinterpret_cast<const q35_u32x2 *>(blk + 24 + 32 * v);
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            const q35_u32x2 x = cp[m];
-            c[i][v][2 * m] = x[0];
-            c[i][v][2 * m + 1] = x[1];
-          }
+          const q35_u32x2 x = *reinterpret_cast<const q35_u32x2 *>(blk + 24 + 32 * v + 8 * t);
+          c[i][v][0] = x[0];
+          c[i][v][1] = x[1];
         } else {
-          // scale, sum, qs[32] from byte 6, pad: five aligned 8-byte words
-          const q35_u32x2 *bp = reinterpret_cast<const q35_u32x2 *>(a.act + (static_cast<size_t>(v) * a.nb + b) * 40);
-          uint32_t d[10];
-#pragma unroll
-          for (int m = 0; m < 5; ++m) {
-            const q35_u32x2 x = bp[m];
-            d[2 * m] = x[0];
-            d[2 * m + 1] = x[1];
-          }
-          sa[i][v] = __uint_as_float(d[0]);
-#pragma unroll
-          for (int m = 0; m < 8; ++m) c[i][v][m] = (d[m + 1] >> 16) | (d[m + 2] << 16);
+          // scale, sum, qs[32] from byte 6: the word before the eight codes, then two
+          const uint8_t *blk = a.act + (static_cast<size_t>(v) * a.nb + b) * 40;
+          sa[i][v] = *reinterpret_cast<const float *>(blk);
+          const q35_u32x2 x = *reinterpret_cast<const q35_u32x2 *>(blk + 8 + 8 * t);
+          c[i][v][0] = *reinterpret_cast<const uint32_t *>(blk + 4 + 8 * t);
+          c[i][v][1] = x[0];
+          c[i][v][2] = x[1];
         }
       }
     }
+  };
+  load(0);
+  for (int b0 = 0; b0 < a.nb; b0 += kPass) {
+    const int n = min(kPass, a.nb - b0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int bl = j + 8 * (wave + 4 * i);
+    for (int i = 0; i < STEPS; ++i) {
+      const int bl = j + 8 * wave + kMvStep * i;
+      const float dw = half_bits_to_float(dh[i]);
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        int acc = 0;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          acc = Q35_SDOT4(wq[i][t] & 0x0f0f0f0fu, c[i][v][2 * t], acc);
-          acc = Q35_SDOT4((wq[i][t] >> 4) & 0x0f0f0f0fu, c[i][v][2 * t + 1], acc);
+        uint32_t lo = c[i][v][0], hi = c[i][v][1];
+        if constexpr (!X4) {
+          lo = (lo >> 16) | (hi << 16);
+          hi = (hi >> 16) | (c[i][v][2] << 16);
         }
+        const int corr = Q35_SDOT4(0xF8F8F8F8u, hi, Q35_SDOT4(0xF8F8F8F8u, lo, 0));
+        int p[4];
 #pragma unroll
-        for (int m = 0; m < 8; ++m) acc = Q35_SDOT4(0xF8F8F8F8u, c[i][v][m], acc);
-        if (bl < n) fs[v][r][bl] = q35_f32x2{static_cast<float>(acc), dw[i] * sa[i][v]};
+        for (int k = 0; k < 4; ++k)
+          p[k] = Q35_SDOT4((wq[i][k] >> 4) & 0x0f0f0f0fu, hi, Q35_SDOT4(wq[i][k] & 0x0f0f0f0fu, lo, corr));
+        // lane t keeps row 4h + t: the odd lanes of a pair take rows 1 and 3,
+        // then the upper lanes of a pair of pairs rows 2 and 3
+        const bool t0 = (t & 1) != 0, t1 = (t & 2) != 0;
+        const int a0 = (t0 ? p[1] : p[0]) + q35_row_xor_i(t0 ? p[0] : p[1], 1);
+        const int a1 = (t0 ? p[3] : p[2]) + q35_row_xor_i(t0 ? p[2] : p[3], 1);
+        const int dot = (t1 ? a1 : a0) + q35_row_xor_i(t1 ? a0 : a1, 2);
+        if (bl < n) fs[v][r][bl] = q35_f32x2{static_cast<float>(dot), dw * sa[i][v]};
       }
     }
     lds_barrier();
+    if (b0 + kPass < a.nb) load(b0 + kPass);
     if (tid < 8 * NV) {
       const int rr = tid & 7, v = tid >> 3;
+#pragma unroll 8
       for (int bl = 0; bl < n; ++bl) {
         const q35_f32x2 p = fs[v][rr][bl];
         res = fmaf(p[0], p[1], res);
@@ -124,16 +137,33 @@ hipError_t launch_dot4_matvec(const q35_q4_0_block_x8 *w, const void *act, bool 
   a.out = out;
   a.stride = stride;
   const dim3 grid(rows / 8), block(kMvThreads);
+  // as many steps per pass as the row has blocks, up to four
+#define Q35_MV(NV, X)                                                                                          \
+  switch (std::min(4, (nb + kMvStep - 1) / kMvStep)) {                                                         \
+    case 1: Q35_LAUNCH((dot4_matvec_kernel<NV, X, 1>), grid, block, 0, stream, a); break;                      \
+    case 2: Q35_LAUNCH((dot4_matvec_kernel<NV, X, 2>), grid, block, 0, stream, a); break;                      \
+    case 3: Q35_LAUNCH((dot4_matvec_kernel<NV, X, 3>), grid, block, 0, stream, a); break;                      \
+    default: Q35_LAUNCH((dot4_matvec_kernel<NV, X, 4>), grid, block, 0, stream, a); break;                     \
+  }
   if (x4) {
-    Q35_LAUNCH((dot4_matvec_kernel<4, true>), grid, block, 0, stream, a);
+    Q35_MV(4, true)
   } else {
     switch (count) {
-      case 1: Q35_LAUNCH((dot4_matvec_kernel<1, false>), grid, block, 0, stream, a); break;
-      case 2: Q35_LAUNCH((dot4_matvec_kernel<2, false>), grid, block, 0, stream, a); break;
-      case 3: Q35_LAUNCH((dot4_matvec_kernel<3, false>), grid, block, 0, stream, a); break;
-      default: Q35_LAUNCH((dot4_matvec_kernel<4, false>), grid, block, 0, stream, a); break;
+      case 1:
+        // rows past four steps in passes of up to nine (the 4B down projection's
+        // 288 blocks are one pass: 8.0 us against 10.5 in passes of four)
+        if (nb > 4 * kMvStep) {
+          Q35_LAUNCH((dot4_matvec_kernel<1, false, 9>), grid, block, 0, stream, a);
+        } else {
+          Q35_MV(1, false)
+        }
+        break;
+      case 2: Q35_MV(2, false) break;
+      case 3: Q35_MV(3, false) break;
+      default: Q35_MV(4, false) break;
     }
   }
+#undef Q35_MV
   return hipGetLastError();
 }
 

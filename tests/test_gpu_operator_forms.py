@@ -1,6 +1,6 @@
 """Operator forms at the sizes where their launches change shape: run and
 vector edges of the convolution, candidate lists with ties and few tokens,
-batches of the direct GEMM.
+batches of the direct GEMM, block counts of the GEMV's passes.
 Each against the oracle's token-by-token or single-value form, within the
 rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
@@ -120,3 +120,28 @@ def test_direct_gemm_forms(q, ctx, orc, rows, blocks, tokens):
     np.testing.assert_array_equal(x4[:tokens].view(np.uint32), got.view(np.uint32))
     few = run(q.q4_dot4_matmul_x1, x1_blocks(codes[:5], scales[:5]), 5, rows)
     np.testing.assert_array_equal(few.view(np.uint32), got[:5].view(np.uint32))
+
+
+@pytest.mark.parametrize("blocks", [1, 31, 32, 33, 64, 65, 97, 128, 129, 257, 288, 289, 577])
+def test_gemv_passes(q, ctx, orc, blocks):
+    """Every step count and pass boundary of the GEMV, one to four vectors:
+    the bits of the exact-mode GEMM (one block-order chain per output)."""
+    rng = np.random.default_rng(blocks)
+    rows, cols = 24, 32 * blocks
+    dm = ctx.array(orc.dot4_pack(orc.random_q4_blocks(rng, rows, cols), rows, blocks))
+    x4 = np.zeros((1, blocks), np.dtype([("s", "<f4", 4), ("sum", "<i2", 4), ("q", "i1", (4, 32))]))
+    x4["s"] = rng.uniform(0.001, 0.02, size=(1, blocks, 4))
+    x4["q"] = rng.integers(-127, 128, size=(1, blocks, 4, 32))
+    x4["sum"] = x4["q"].astype(np.int32).sum(-1)
+    x1 = np.zeros((4, blocks), np.dtype([("s", "<f4"), ("sum", "<i2"), ("q", "i1", 32), ("pad", "<i2")]))
+    x1["s"], x1["sum"], x1["q"] = x4["s"][0].T, x4["sum"][0].T, x4["q"][0].transpose(1, 0, 2)
+    d4, d1, out = ctx.array(x4.view(np.uint8)), ctx.array(x1.view(np.uint8)), ctx.array(shape=(4, rows), dtype=np.float32)
+    print(f"GEMV {blocks} blocks", flush=True)
+    q.q4_dot4_matmul(ctx, dm, d4, out, rows, 4, blocks, rows, exact=True)
+    want = out.download().view(np.uint32)
+    q.q4_dot4_matmul(ctx, dm, d4, out, rows, 4, blocks, rows)
+    np.testing.assert_array_equal(out.download().view(np.uint32), want)
+    for n in (1, 2, 3, 4):
+        dst = ctx.array(shape=(n, rows), dtype=np.float32)
+        q.q4_dot4_matmul_x1(ctx, dm, d1, dst, rows, n, blocks, rows)
+        np.testing.assert_array_equal(dst.download().view(np.uint32), want[:n])
