@@ -73,6 +73,30 @@ __global__ __launch_bounds__(kPrepThreads) void prep_kernel(PrepArgs a) {
   h128_quantize_lanes<kPrepLanes>(v, t, blk, nb, a.h128, a.seed, o, active);
 }
 
+// X4 outputs (plain rows, tokens % 4 == 0): one wavefront per (four tokens,
+// 128-column block), 16 lanes per token, so that it writes the four X4 blocks
+// -- 608 contiguous bytes -- whole. What bounds it is memory: with a token per
+// half wavefront the 32-byte pieces of a block came from four workgroups, and
+// 2048 x 9216 took 26.3-29.9 us (3.3-3.7 TB/s); this form 19.6 us (5.0 TB/s).
+__global__ __launch_bounds__(kPrepThreads) void prep_x4_kernel(PrepArgs a) {
+  const int K = a.K, nblk = K >> 7, lane = threadIdx.x & 63;
+  const int groups = (a.tokens >> 2) * nblk;
+  const int group = static_cast<int>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (group >= groups) return;  // whole wavefront
+  const int t4 = group / nblk, blk = group - t4 * nblk, t = 4 * t4 + (lane >> 4);
+  const q35_f32x4 *src = reinterpret_cast<const q35_f32x4 *>(a.x + static_cast<size_t>(t) * a.x_stride + blk * 128 + 8 * (lane & 15));
+  const q35_f32x4 lo = src[0], hi = src[1];
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = lo[e];
+    v[4 + e] = hi[e];
+  }
+  QuantOut o;
+  o.x4 = a.x4;
+  h128_quantize_row16(v, t, blk, K >> 5, a.h128, a.seed, o, true);
+}
+
 // Residual update + RMSNorm + preparation, one workgroup (256 threads) per
 // token. Thread i owns the float4 columns 4i + 1024k; the residual and the
 // split partial rows of a column batch are loaded before the ordered sum.
@@ -318,6 +342,10 @@ hipError_t launch_prep(const PrepArgs &a, hipStream_t stream) {
       case 8: Q35_LAUNCH((prep_kernel<kPrepSiluMul, 8>), grid, block, 0, stream, a); break;
       default: return hipErrorInvalidValue;
     }
+  } else if (a.x4 != nullptr && a.x1 == nullptr && a.codes == nullptr && a.y_out == nullptr && a.tokens % 4 == 0) {
+    // four wavefronts per workgroup once the launch has some for every compute unit
+    const int groups = a.tokens / 4 * (a.K >> 7), waves = groups >= 4096 ? 4 : 1;
+    Q35_LAUNCH((prep_x4_kernel), dim3((groups + waves - 1) / waves), dim3(64 * waves), 0, stream, a);
   } else {
     Q35_LAUNCH((prep_kernel<kPrepPlain, 1>), grid, block, 0, stream, a);
   }

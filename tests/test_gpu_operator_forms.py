@@ -1,6 +1,7 @@
 """Operator forms at the sizes where their launches change shape: run and
 vector edges of the convolution, candidate lists with ties and few tokens,
-batches of the direct GEMM, block counts of the GEMV's passes.
+batches of the direct GEMM, block counts of the GEMV's passes,
+wavefront tails of the X4 preparation.
 Each against the oracle's token-by-token or single-value form, within the
 rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
@@ -145,3 +146,32 @@ def test_gemv_passes(q, ctx, orc, blocks):
         dst = ctx.array(shape=(n, rows), dtype=np.float32)
         q.q4_dot4_matmul_x1(ctx, dm, d1, dst, rows, n, blocks, rows)
         np.testing.assert_array_equal(dst.download().view(np.uint32), want[:n])
+
+
+@pytest.mark.parametrize("tokens,cols", [(4, 128), (8, 384), (12, 640), (5468, 384)])
+@pytest.mark.parametrize("h128", [True, False])
+def test_x4_preparation_equals_rows(q, ctx, tokens, cols, h128):
+    """X4 blocks (one wavefront per four tokens and 128 columns, alone or four
+    to a workgroup with a tail) hold the bytes of the rows prepared one by one."""
+    rng = np.random.default_rng(tokens + cols)
+    x = rng.standard_normal((tokens, cols)).astype(np.float32)
+    x[1] = 0.0
+    nb = cols // 32
+    x4t = np.dtype([("s", "<f4", 4), ("sum", "<i2", 4), ("q", "i1", (4, 32))])
+    x1t = np.dtype([("s", "<f4"), ("sum", "<i2"), ("q", "i1", 32), ("pad", "<i2")])
+    d4 = ctx.array(shape=(tokens // 4, nb, 152), dtype=np.uint8)
+    print(f"X4 preparation {tokens} x {cols} h128 {h128}", flush=True)
+    if h128:
+        q.q4_h128_prepare_activations_4(ctx, ctx.array(x), d4, tokens, cols)
+    else:
+        q.q8_0_quantize_vectors_4(ctx, ctx.array(x), d4, tokens, nb)
+    got = d4.download().view(x4t).reshape(tokens // 4, nb)
+    for r in sorted({0, 1, 2, 3, tokens // 2, tokens - 2, tokens - 1}):
+        d1 = ctx.array(shape=(nb, 40), dtype=np.uint8)
+        if h128:
+            q.q4_h128_prepare_activation_1(ctx, ctx.array(x[r:r + 1]), d1, cols)
+        else:
+            q.q8_0_quantize_vector_1(ctx, ctx.array(x[r:r + 1]), d1, nb)
+        one = d1.download().view(x1t).reshape(nb)
+        for f in ("s", "sum", "q"):
+            np.testing.assert_array_equal(got[r // 4][f][:, r % 4], one[f])
