@@ -232,13 +232,12 @@ __device__ __forceinline__ q35_f16x8 v_operand(const VOps &v, int ks, int j) {
 // tokens per page), so one page-table entry serves a lane's 8 value tokens
 // (2 entry loads per thread instead of 16).
 template <int QPK, bool GROUPS>
-__global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_kernel(AttnArgs a) {
+__device__ __forceinline__ void attention_chunk(const AttnArgs &a, int sp, int g, int ord) {
   constexpr int kQStride = kHeadDim + 4;  // floats per staged query row (rows start on different banks)
   __shared__ __align__(16) float qs[QPK * kQStride];
   __shared__ __align__(16) float pl[16 * kPStride];
   __shared__ float tmax[4][16], tsum[4][16];
-  const int sp = blockIdx.x, g = blockIdx.y;
-  const int ord = static_cast<int>(blockIdx.z);  // partial rows are indexed by the ordinal
+  // partial rows are indexed by the ordinal
   const int r = a.row_list != nullptr ? a.row_list[ord] : ord;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int t0 = sp * kChunkTokens;
@@ -280,6 +279,9 @@ __global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_kernel(Attn
   const bool kin = kt < n;
   const uint16_t *krow = a.k_pool + ((static_cast<size_t>(kin ? pk : pfirst) << pshift) + ((kin ? t0 + kt : t0) & pmask)) * kvw +
                          static_cast<size_t>(g) * kHeadDim + 8 * (lane >> 4);
+  // streamed (non-temporal): cached key loads are faster on a pool that is
+  // read again and again (64 rows, contexts 128 to 8192: 252 against 271 us a
+  // call) but slower right after it was written (310 against 268)
   q35_u32x4 kraw[8];
 #pragma unroll
   for (int kk = 0; kk < 8; ++kk) kraw[kk] = Q35_LOAD_NT(reinterpret_cast<const q35_u32x4 *>(krow + 32 * kk));
@@ -361,6 +363,38 @@ __global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_kernel(Attn
     a.part_ml[hs * 2] = mx;
     a.part_ml[hs * 2 + 1] = ((tsum[0][lane] + tsum[1][lane]) + tsum[2][lane]) + tsum[3][lane];
   }
+}
+
+template <int QPK, bool GROUPS>
+__global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_kernel(AttnArgs a) {
+  attention_chunk<QPK, GROUPS>(a, static_cast<int>(blockIdx.x), static_cast<int>(blockIdx.y),
+                               static_cast<int>(blockIdx.z));
+}
+
+// The same over exactly the chunks that rows row0 .. row0 + n - 1 have, where
+// the host knows their context lengths: first[i] is the number of chunks
+// before row i, so workgroup x finds its row by bisection (scalar loads of the
+// kernel arguments). A grid as wide as the longest context launches a
+// workgroup for every chunk a shorter row lacks, which costs a dispatch and a
+// round trip before it returns (64 rows, contexts 128 to 8192: half of them;
+// 16 rows of 64 to 4096: 43.5 -> 35.0 us a call with the lengths read back
+// through pinned memory, 1 row of 8000: 38.0 -> 30.6).
+constexpr int kRaggedRows = 64;
+struct RaggedRows {
+  int n, row0;
+  int first[kRaggedRows + 1];
+};
+
+template <int QPK, bool GROUPS>
+__global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_ragged_kernel(AttnArgs a, RaggedRows rows) {
+  const int x = static_cast<int>(blockIdx.x);
+  int lo = 0, hi = rows.n;  // first[lo] <= x < first[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (rows.first[mid] <= x) lo = mid;
+    else hi = mid;
+  }
+  attention_chunk<QPK, GROUPS>(a, x - rows.first[lo], static_cast<int>(blockIdx.y), rows.row0 + lo);
 }
 
 // Prefill and packed steps: one workgroup per (tile of up to kAttnTileRows
@@ -780,6 +814,16 @@ hipError_t launch_attn_prep(const AttnPrepArgs &a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+static RaggedRows ragged_rows(const AttnArgs &a, int row0) {
+  RaggedRows rows;
+  rows.row0 = row0;
+  rows.n = std::min(kRaggedRows, a.batch - row0);
+  rows.first[0] = 0;
+  for (int i = 0; i < rows.n; ++i)
+    rows.first[i + 1] = rows.first[i] + (a.host_lens[row0 + i] + kChunkTokens - 1) / kChunkTokens;
+  return rows;
+}
+
 hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   if (a.batch <= 0) return hipSuccess;
   if (a.head_dim != kHeadDim || a.heads % a.kv_heads != 0 || a.split_tokens != kChunkTokens)
@@ -790,13 +834,29 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   // tiled: the prompt tiles, then the one-row segments' rows as decode rows
   const int decode_rows = tiled ? a.row_count : a.batch;
   if (tiled && a.tiles > 0 && (a.prompt_o == nullptr || a.prompt_ml == nullptr)) return hipErrorInvalidValue;
+  // known context lengths: only the chunks that the rows have, unless that
+  // saves less than a tenth of the grid
+  long long chunks = 0;
+  if (!tiled && a.row_list == nullptr && a.host_lens != nullptr)
+    for (int r = 0; r < a.batch; ++r) chunks += (a.host_lens[r] + kChunkTokens - 1) / kChunkTokens;
+  const bool ragged = chunks > 0 && 10 * chunks < 9LL * gs * a.batch;
 #define Q35_ATTN(Q)                                                                                    \
   if (tiled && a.tiles > 0)                                                                            \
     Q35_LAUNCH((attention_flash_kernel<Q>), dim3(a.tiles, a.kv_heads), dim3(128 * (Q)), 0, stream, a); \
-  if (decode_rows > 0 && a.page_tokens >= 8)                                                          \
-    Q35_LAUNCH((attention_kernel<Q, true>), dim3(gs, a.kv_heads, decode_rows), dim3(256), 0, stream, a); \
-  else if (decode_rows > 0)                                                                            \
-    Q35_LAUNCH((attention_kernel<Q, false>), dim3(gs, a.kv_heads, decode_rows), dim3(256), 0, stream, a);
+  if (ragged) {                                                                                        \
+    for (int row0 = 0; row0 < a.batch; row0 += kRaggedRows) {                                          \
+      RaggedRows rows = ragged_rows(a, row0);                                                          \
+      const dim3 grid(rows.first[rows.n], a.kv_heads);                                                 \
+      if (a.page_tokens >= 8)                                                                          \
+        Q35_LAUNCH((attention_ragged_kernel<Q, true>), grid, dim3(256), 0, stream, a, rows);           \
+      else                                                                                             \
+        Q35_LAUNCH((attention_ragged_kernel<Q, false>), grid, dim3(256), 0, stream, a, rows);          \
+    }                                                                                                  \
+  } else if (decode_rows > 0 && a.page_tokens >= 8) {                                                  \
+    Q35_LAUNCH((attention_kernel<Q, true>), dim3(gs, a.kv_heads, decode_rows), dim3(256), 0, stream, a);  \
+  } else if (decode_rows > 0) {                                                                        \
+    Q35_LAUNCH((attention_kernel<Q, false>), dim3(gs, a.kv_heads, decode_rows), dim3(256), 0, stream, a); \
+  }
   switch (qpk) {
     case 1: Q35_ATTN(1) break;
     case 2: Q35_ATTN(2) break;

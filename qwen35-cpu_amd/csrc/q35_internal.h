@@ -21,6 +21,8 @@ struct Context {
   std::string arch;
   std::string error;
   hipEvent_t t0 = nullptr, t1 = nullptr;
+  int32_t *host_lens = nullptr;  // pinned, grow-only: context lengths read back by the attention entry point
+  size_t host_lens_capacity = 0;
 };
 
 int set_error(Context *ctx, int status, const std::string &message);
@@ -428,6 +430,7 @@ struct AttnArgs {
   int max_pages = 0, page_tokens = 0;
   const int32_t *seq_lens = nullptr;     // either seq_lens or positions(+1)
   const int32_t *positions = nullptr;
+  const int32_t *host_lens = nullptr;    // host copy of seq_lens, where the caller has one (read at launch)
   int batch = 0, heads = 0, kv_heads = 0, head_dim = 0;
   float scale = 0.0625F;
   int split_tokens = 64, max_splits = 1;  // split_tokens must be kAttnChunkTokens

@@ -112,6 +112,7 @@ extern "C" void q35_context_destroy(q35_context *ctx) {
   }
   (void)hipEventDestroy(ctx->t0);
   (void)hipEventDestroy(ctx->t1);
+  if (ctx->host_lens != nullptr) (void)hipHostFree(ctx->host_lens);
   if (ctx->own_stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
 }
@@ -518,6 +519,15 @@ extern "C" int q35_gated_delta_net_update_batch(q35_context *ctx, float *const *
 }
 
 // ================================================================ attention
+namespace q35 {
+namespace {
+__global__ void copy_i32_kernel(const int32_t *src, int32_t *dst, size_t n) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+}  // namespace
+}  // namespace q35
+
 extern "C" int q35_attention_decode_paged(q35_context *ctx, const float *q, const float *gates,
                                           const uint16_t *k_pool, const uint16_t *v_pool,
                                           const int32_t *page_table, size_t max_pages,
@@ -529,11 +539,28 @@ extern "C" int q35_attention_decode_paged(q35_context *ctx, const float *q, cons
       (page_tokens & (page_tokens - 1)) != 0 || page_tokens > (1u << 20))
     return set_error(ctx, Q35_ERR_UNSUPPORTED,
                      "attention needs head_dim 256, heads % kv_heads == 0 and a power-of-two page size");
-  std::vector<int32_t> lens(batch);
-  Q35_HIP_TRY(ctx, hipMemcpyAsync(lens.data(), seq_lens, batch * 4, hipMemcpyDeviceToHost, ctx->stream));
+  // the lengths come back into pinned memory, written by a small kernel: a
+  // copy to pageable memory goes through the runtime's staging buffer and waits
+  // for it, and one to pinned memory wakes a copy engine
+  if (ctx->host_lens_capacity < batch) {
+    if (ctx->host_lens != nullptr) (void)hipHostFree(ctx->host_lens);
+    ctx->host_lens = nullptr;
+    ctx->host_lens_capacity = 0;
+    void *p = nullptr;
+    Q35_HIP_TRY(ctx, hipHostMalloc(&p, batch * 4));
+    ctx->host_lens = static_cast<int32_t *>(p);
+    ctx->host_lens_capacity = batch;
+  }
+  const int32_t *lens = ctx->host_lens;
+  void *mapped = nullptr;
+  Q35_HIP_TRY(ctx, hipHostGetDevicePointer(&mapped, ctx->host_lens, 0));
+  Q35_LAUNCH((q35::copy_i32_kernel), static_cast<unsigned>((batch + 255) / 256), 256, 0, ctx->stream, seq_lens,
+             static_cast<int32_t *>(mapped), batch);
+  Q35_HIP_TRY(ctx, hipGetLastError());
   Q35_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   int max_len = 1;
-  for (auto l : lens) {
+  for (size_t r = 0; r < batch; ++r) {
+    const int32_t l = lens[r];
     if (l <= 0 || static_cast<size_t>(l) > max_pages * page_tokens)
       return set_error(ctx, Q35_ERR_INVALID, "sequence length outside the page table");
     max_len = std::max(max_len, l);
@@ -546,6 +573,7 @@ extern "C" int q35_attention_decode_paged(q35_context *ctx, const float *q, cons
   a.max_pages = static_cast<int>(max_pages);
   a.page_tokens = static_cast<int>(page_tokens);
   a.seq_lens = seq_lens;
+  a.host_lens = lens;
   a.batch = static_cast<int>(batch);
   a.heads = heads;
   a.kv_heads = kv_heads;

@@ -1,7 +1,8 @@
 """Operator forms at the sizes where their launches change shape: run and
 vector edges of the convolution, candidate lists with ties and few tokens,
 batches of the direct GEMM, block counts of the GEMV's passes,
-wavefront tails of the X4 preparation.
+wavefront tails of the X4 preparation,
+ragged attention grids.
 Each against the oracle's token-by-token or single-value form, within the
 rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
@@ -175,3 +176,38 @@ def test_x4_preparation_equals_rows(q, ctx, tokens, cols, h128):
         one = d1.download().view(x1t).reshape(nb)
         for f in ("s", "sum", "q"):
             np.testing.assert_array_equal(got[r // 4][f][:, r % 4], one[f])
+
+
+@pytest.mark.parametrize("batch,page_tokens,lens", [
+    (2, 16, (1, 700)), (3, 4, (130, 1, 64)), (64, 16, None), (65, 16, None), (130, 8, None)])
+def test_ragged_attention_equals_rows_alone(q, ctx, batch, page_tokens, lens):
+    """Rows of unequal contexts in one call (the grid of exactly their chunks,
+    in groups of 64 rows) give the bits of each row called alone."""
+    rng = np.random.default_rng(batch)
+    heads, kv, hd = 4, 2, 256
+    lens = np.asarray(lens if lens is not None else rng.integers(1, 500, size=batch), np.int32)
+    lens[-1] = max(lens[-1], 641)  # one long row: the others leave most of the full grid idle
+    need = (lens + page_tokens - 1) // page_tokens
+    pool = rng.standard_normal((2, int(need.sum()), page_tokens, kv, hd)).astype(np.float16).view(np.uint16)
+    table = np.zeros((batch, need.max()), np.int32)
+    perm, at = rng.permutation(int(need.sum())), 0
+    for r in range(batch):
+        table[r, :need[r]] = perm[at:at + need[r]]
+        at += need[r]
+    qv, gates = rng.standard_normal((2, batch, heads * hd)).astype(np.float32)
+    dk, dv = ctx.array(pool[0]), ctx.array(pool[1])
+
+    def call(rows):
+        out = ctx.array(shape=(len(rows), heads * hd), dtype=np.float32)
+        q.attention_decode_paged(ctx, ctx.array(qv[rows]), ctx.array(gates[rows]), dk, dv, ctx.array(table[rows]),
+                                 table.shape[1], ctx.array(lens[rows]), page_tokens, out, len(rows), heads, kv, hd,
+                                 1.0 / 16.0)
+        return out.download().view(np.uint32)
+
+    print(f"ragged attention batch {batch} page {page_tokens}", flush=True)
+    together = call(np.arange(batch))
+    for r in sorted({0, 1, batch // 2, min(63, batch - 1), min(64, batch - 1), batch - 1}):
+        np.testing.assert_array_equal(call(np.array([r]))[0], together[r])
+    with pytest.raises(q.Q35Error):
+        lens[0] = table.shape[1] * page_tokens + 1
+        call(np.arange(batch))
