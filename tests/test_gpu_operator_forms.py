@@ -2,7 +2,7 @@
 vector edges of the convolution, candidate lists with ties and few tokens,
 batches of the direct GEMM, block counts of the GEMV's passes,
 wavefront tails of the X4 preparation,
-ragged attention grids.
+ragged attention grids, the greedy head's counts.
 Each against the oracle's token-by-token or single-value form, within the
 rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
@@ -211,3 +211,29 @@ def test_ragged_attention_equals_rows_alone(q, ctx, batch, page_tokens, lens):
     with pytest.raises(q.Q35Error):
         lens[0] = table.shape[1] * page_tokens + 1
         call(np.arange(batch))
+
+
+@pytest.mark.parametrize("blocks", [1, 12, 13, 16, 33])
+@pytest.mark.parametrize("rows,vectors", [(8, 4), (72, 12), (200, 16), (520, 20), (1000, 36)])
+def test_head_counts_of_the_best_rows(q, ctx, orc, rows, blocks, vectors):
+    """Greedy head with the best rows of each token counted, so that a count
+    read for another row or token changes the winner: fewer than four chunks
+    of four blocks (counts read at a group's end) and more (read ahead), one
+    and several token tiles, ragged row groups. Exact index and value."""
+    rng = np.random.default_rng(rows * 100 + blocks)
+    packed = orc.dot4_pack(orc.random_q4_blocks(rng, rows, blocks * 32), rows, blocks)
+    act = orc.q8_quantize_4(rng.standard_normal((vectors, blocks * 32)).astype(np.float32))
+    adj = orc.dot4_matmul(packed, act, rows, vectors, blocks).copy()
+    pen = np.where(np.arange(vectors) % 4 == 3, 1.0, 1.5).astype(np.float32)
+    counts = np.zeros((vectors, rows), np.int32)
+    for v in range(vectors):
+        counts[v, np.argsort(adj[v])[-1 - v % 4:]] = 1 + v
+        m = (counts[v] > 0) & (pen[v] > 1)
+        adj[v, m] = np.where(adj[v, m] > 0, adj[v, m] / pen[v], adj[v, m] * pen[v])
+    want = adj.argmax(1)
+    idx = ctx.array(shape=(vectors,), dtype=np.int32)
+    val = ctx.array(shape=(vectors,), dtype=np.float32)
+    q.q4_dot4_argmax_batch(ctx, ctx.array(packed), ctx.array(act), ctx.array(counts), ctx.array(pen), rows, vectors,
+                           blocks, idx, val)
+    np.testing.assert_array_equal(idx.download(), want)
+    np.testing.assert_array_equal(val.download(), adj[np.arange(vectors), want])
