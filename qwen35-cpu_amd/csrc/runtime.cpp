@@ -271,11 +271,37 @@ size_t dot4_matmul_scratch_bytes(int rows, int nb, int chunk, bool argmax, int c
   return code_bytes + scale_bytes + cand_bytes + part_bytes;
 }
 
+// Whether plain outputs run the direct GEMM, which writes outputs while other
+// workgroups still read the activations and weights: where it fits, unless
+// they share memory. (The other forms copy the activations to scratch first,
+// so outputs may overlap them.)
+static bool dot4_matmul_direct(const Context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_block_x4 *x4,
+                               const q35_q8_0_block_x1 *x1, const float *out, size_t rows, size_t vectors,
+                               size_t blocks, size_t stride) {
+  if (!gemm_direct_fits(static_cast<int>(rows), static_cast<int>(blocks), vectors, ctx->cu_count)) return false;
+  const uintptr_t o0 = reinterpret_cast<uintptr_t>(out), o1 = o0 + ((vectors - 1) * stride + rows) * sizeof(float);
+  const auto apart = [&](const void *p, size_t bytes) {
+    const uintptr_t p0 = reinterpret_cast<uintptr_t>(p);
+    return p0 >= o1 || o0 >= p0 + bytes;
+  };
+  return apart(m, rows / 8 * blocks * sizeof(*m)) &&
+         (x4 != nullptr ? apart(x4, (vectors + 3) / 4 * blocks * sizeof(*x4)) : apart(x1, vectors * blocks * sizeof(*x1)));
+}
+
+// Whether a call needs no scratch: plain outputs of the GEMV or the direct GEMM.
+static bool dot4_matmul_scratch_free(const Context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_block_x4 *x4,
+                                     const q35_q8_0_block_x1 *x1, const float *out, const int32_t *dots, size_t rows,
+                                     size_t vectors, size_t blocks, size_t stride, bool exact, const int32_t *index) {
+  return out != nullptr && dots == nullptr && index == nullptr && !exact &&
+         (vectors <= static_cast<size_t>(kMatvecMaxVectors) ||
+          dot4_matmul_direct(ctx, m, x4, x1, out, rows, vectors, blocks, stride));
+}
+
 // Runs the GEMM over `vectors` tokens, `chunk` (a multiple of 16; above
-// kMaxTokens only for plain outputs, which then run the dense GEMM) at a time, from X4 or X1 activations, with the activation
-// layout, candidates and split partials in `scratch` (at least
-// dot4_matmul_scratch_bytes). `exact` forces the single-wave fma chain per
-// row. With `index` set it runs the greedy head instead (penalty + argmax per
+// kMaxTokens only for plain outputs, which then run the dense GEMM) at a time,
+// from X4 or X1 activations, with the activation layout, candidates and split
+// partials in `scratch` (at least dot4_matmul_scratch_bytes; unused where
+// dot4_matmul_scratch_free). `exact` forces the single-wave fma chain per row. With `index` set it runs the greedy head instead (penalty + argmax per
 // vector). The K split depends on rows and blocks only, so every chunk size
 // gives the same bits.
 int dot4_matmul_run(Context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_block_x4 *x4,
@@ -283,22 +309,20 @@ int dot4_matmul_run(Context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_blo
                     size_t blocks, size_t stride, bool exact, int32_t *index, float *value, const int32_t *counts,
                     const float *penalties, void *scratch, size_t chunk) {
   const int nb = static_cast<int>(blocks);
-  if (out != nullptr && dots == nullptr && index == nullptr && !exact && vectors <= kMatvecMaxVectors) {
+  if (dot4_matmul_scratch_free(ctx, m, x4, x1, out, dots, rows, vectors, blocks, stride, exact, index)) {
+    const void *act = x4 != nullptr ? static_cast<const void *>(x4) : x1;
     // one to four vectors: the single-launch dot4 GEMV (bit-exact chains)
-    const hipError_t e = launch_dot4_matvec(m, x4 != nullptr ? static_cast<const void *>(x4) : x1, x4 != nullptr,
-                                            static_cast<int>(vectors), static_cast<int>(rows), nb, out,
-                                            static_cast<long long>(stride), ctx->stream);
-    if (e != hipSuccess) return hip_error(ctx, e, "dot4 GEMV kernel");
+    const bool gemv = vectors <= static_cast<size_t>(kMatvecMaxVectors);
+    const hipError_t e = gemv ? launch_dot4_matvec(m, act, x4 != nullptr, static_cast<int>(vectors),
+                                                   static_cast<int>(rows), nb, out, static_cast<long long>(stride),
+                                                   ctx->stream)
+                              : launch_gemm_direct(m, act, x4 != nullptr, static_cast<int>(rows), nb,
+                                                   static_cast<int>(vectors), out, static_cast<long long>(stride),
+                                                   ctx->cu_count, ctx->stream);
+    if (e != hipSuccess) return hip_error(ctx, e, gemv ? "dot4 GEMV kernel" : "direct DOT4 GEMM kernel");
     return Q35_OK;
   }
-  if (out != nullptr && dots == nullptr && index == nullptr && !exact &&
-      gemm_direct_fits(static_cast<int>(rows), nb, vectors, ctx->cu_count)) {
-    const hipError_t e = launch_gemm_direct(m, x4 != nullptr ? static_cast<const void *>(x4) : x1, x4 != nullptr,
-                                            static_cast<int>(rows), nb, static_cast<int>(vectors), out,
-                                            static_cast<long long>(stride), ctx->cu_count, ctx->stream);
-    if (e != hipSuccess) return hip_error(ctx, e, "direct DOT4 GEMM kernel");
-    return Q35_OK;
-  }
+  if (scratch == nullptr) return set_error(ctx, Q35_ERR_INVALID, "DOT4 GEMM without scratch");
   const size_t tiles = (chunk + 15) / 16;
   const size_t code_bytes = align256(tiles * 64 * static_cast<size_t>(nb) * sizeof(uint64_t));
   const size_t scale_bytes = align256(tiles * 16 * static_cast<size_t>(nb) * sizeof(float));
@@ -384,11 +408,7 @@ int matmul_entry(q35_context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_bl
                      vectors > static_cast<size_t>(kMaxTokens);
   const size_t chunk = dense ? std::min<size_t>((vectors + 15) / 16 * 16, kDenseChunk) : kMaxTokens;
   void *scratch = nullptr;
-  // plain outputs of one to four vectors (the GEMV) or of a batch that the
-  // direct GEMM takes: one launch, no scratch
-  if (out != nullptr && dots == nullptr && index == nullptr && !exact &&
-      (vectors <= static_cast<size_t>(kMatvecMaxVectors) ||
-       gemm_direct_fits(static_cast<int>(rows), static_cast<int>(blocks), vectors, ctx->cu_count)))
+  if (dot4_matmul_scratch_free(ctx, m, x4, x1, out, dots, rows, vectors, blocks, stride, exact, index))
     return dot4_matmul_run(ctx, m, x4, x1, out, dots, rows, vectors, blocks, stride, exact, index, value, counts,
                            penalties, nullptr, chunk);
   st = scratch_get(ctx,

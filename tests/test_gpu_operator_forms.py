@@ -124,6 +124,44 @@ def test_direct_gemm_forms(q, ctx, orc, rows, blocks, tokens):
     np.testing.assert_array_equal(few.view(np.uint32), got[:5].view(np.uint32))
 
 
+class _At:
+    """A place within a device array, as an operator's buffer argument."""
+
+    def __init__(self, array, offset):
+        self.array, self.ptr = array, type(array.ptr)(array.ptr.value + offset)
+
+
+@pytest.mark.parametrize("offset", [0, 160, 1024])
+@pytest.mark.parametrize("rows,blocks,tokens,x1", [(40, 9, 8, False), (40, 9, 7, True), (72, 3, 64, False),
+                                                   (24, 17, 68, False), (24, 2, 67, True)])
+def test_outputs_over_activations(q, ctx, orc, rows, blocks, tokens, x1, offset):
+    """Outputs that share memory with the activations they come from (at its
+    start, ahead of it and within it) are those of separate buffers: such a
+    call reads every activation before its first output is written."""
+    rng = np.random.default_rng(rows + blocks + tokens)
+    dm = ctx.array(orc.dot4_pack(orc.random_q4_blocks(rng, rows, 32 * blocks), rows, blocks))
+    x = rng.standard_normal((tokens, 32 * blocks)).astype(np.float32)
+    act = np.stack([orc.q8_quantize_1(r) for r in x]) if x1 else orc.q8_quantize_4(x)
+    act = np.ascontiguousarray(act).view(np.uint8).ravel()
+    call = q.q4_dot4_matmul_x1 if x1 else q.q4_dot4_matmul
+    stride = rows + 4
+    out_bytes = tokens * stride * 4
+    apart = ctx.array(shape=(tokens, stride), dtype=np.float32)
+    print(f"outputs over activations {rows} rows {blocks} blocks {tokens} tokens at {offset}", flush=True)
+    call(ctx, dm, ctx.array(act), apart, rows, tokens, blocks, stride)
+    want = apart.download()[:, :rows]
+    # (the no-allocation form works in chunks of 64 vectors, so more than one chunk must not overlap)
+    calls = [call] if x1 or tokens > 64 else [call, q.q4_dot4_matmul_noalloc]
+    for a_at, o_at in ((0, offset), (offset, 0)):
+        for f in calls:
+            host = np.zeros(offset + max(act.size, out_bytes), np.uint8)
+            host[a_at:a_at + act.size] = act
+            both = ctx.array(host)
+            f(ctx, dm, _At(both, a_at), _At(both, o_at), rows, tokens, blocks, stride)
+            got = both.download()[o_at:o_at + out_bytes].view(np.float32).reshape(tokens, stride)[:, :rows]
+            np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("blocks", [1, 31, 32, 33, 64, 65, 97, 128, 129, 257, 288, 289, 577])
 def test_gemv_passes(q, ctx, orc, blocks):
     """Every step count and pass boundary of the GEMV, one to four vectors:
