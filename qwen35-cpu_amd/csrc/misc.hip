@@ -59,8 +59,9 @@ __global__ void l2_normalize_kernel(float *x, int width, float eps, float scale)
 // causal_conv1d_silu_f32 (activation.cpp:164-222): kernel-major weights
 // [kernel][channels], the ring of kernel - 1 past inputs per channel in
 // `state` (position p in slot (ring + p) mod (kernel - 1), the call's first
-// token being position 0). The sum of a token: its own input's tap first,
-// then the history oldest first.
+// token being position 0). The sum of a token: the product of its own
+// input's tap, then the history oldest first, one fmaf per tap (written out, so
+// that every form below rounds alike).
 //
 // The history of a token is the call's own input rows except for its first
 // kernel - 1 tokens, so tokens need not run in order: a thread takes V
@@ -130,7 +131,7 @@ __global__ void conv1d_silu_runs_kernel(float *state, int ring, const float *inp
       for (int e = 0; e < V; ++e) {
         sum.v[e] = x[K - 1 + i].v[e] * wk[K - 1].v[e];
 #pragma unroll
-        for (int k = 0; k < K - 1; ++k) sum.v[e] += x[i + k].v[e] * wk[k].v[e];
+        for (int k = 0; k < K - 1; ++k) sum.v[e] = fmaf(x[i + k].v[e], wk[k].v[e], sum.v[e]);
       }
       finish(t0 + i, sum);
     }
@@ -143,7 +144,7 @@ __global__ void conv1d_silu_runs_kernel(float *state, int ring, const float *inp
       for (int k = 0; k < hist; ++k) {
         const ConvVec<V> h = past(t - hist + k), wt = conv_load<V>(w + static_cast<size_t>(k) * channels + c);
 #pragma unroll
-        for (int e = 0; e < V; ++e) sum.v[e] += h.v[e] * wt.v[e];
+        for (int e = 0; e < V; ++e) sum.v[e] = fmaf(h.v[e], wt.v[e], sum.v[e]);
       }
       finish(t, sum);
     }
@@ -165,7 +166,8 @@ __global__ void conv1d_silu_kernel(float *state, int ring, const float *input, l
     const float x = input[t * stride + c];
     float sum = x * w[static_cast<size_t>(hist) * channels + c];
     for (int k = 0; k < hist; ++k)
-      sum += state[static_cast<size_t>((ring + k) % hist) * channels + c] * w[static_cast<size_t>(k) * channels + c];
+      sum = fmaf(state[static_cast<size_t>((ring + k) % hist) * channels + c],
+                 w[static_cast<size_t>(k) * channels + c], sum);
     if (hist) state[static_cast<size_t>(ring) * channels + c] = x;
     out[static_cast<size_t>(t) * channels + c] = silu_times(sum, 1.0F);
     if (hist) ring = (ring + 1) % hist;

@@ -43,6 +43,33 @@ def test_conv1d_runs(q, ctx, orc, batch, ch, kern, begin, end, extra, in_place):
     np.testing.assert_array_equal(dstate.download(), want_state)
 
 
+@pytest.mark.parametrize("kern", [1, 2, 3, 4, 5, 9, 10])
+@pytest.mark.parametrize("batch,ch", [(1, 64), (7, 68), (40, 66), (130, 64)])
+def test_conv1d_bits_do_not_depend_on_the_form(q, ctx, batch, ch, kern):
+    """The sum of a token is one fma chain (its own tap's product, then the
+    history oldest first) in every form: four channels per thread or one, taps
+    in registers or re-read, and the walk through the ring of an in-place call."""
+    rng = np.random.default_rng(batch + ch + kern)
+    hist = kern - 1
+    state = rng.standard_normal((max(hist, 1), ch)).astype(np.float32)
+    x = rng.standard_normal((batch, ch)).astype(np.float32)
+    w = ctx.array((rng.standard_normal((kern, ch)) * 0.5).astype(np.float32))
+
+    def call(place, begin, end):
+        ds, dx = ctx.array(state), ctx.array(x)
+        out = dx if place else ctx.array(np.zeros((batch, ch), np.float32))
+        q.causal_conv1d_silu_f32(ctx, ds, hist // 2 if hist else 0, dx, w, out, ch, kern, batch=batch,
+                                 channel_begin=begin, channel_end=end)
+        return out.download().view(np.uint32)[:, begin:end], ds.download()
+
+    print(f"conv1d forms batch {batch} channels {ch} kernel {kern}", flush=True)
+    want, ring = call(True, 0, ch)
+    for begin, end in ((0, ch), (1, ch - 1)):
+        got, after = call(False, begin, end)
+        np.testing.assert_array_equal(got, want[:, begin:end])
+        np.testing.assert_array_equal(after[:, begin:end], ring[:, begin:end])
+
+
 @pytest.mark.parametrize("vocab,k", [(64, 64), (264, 1), (264, 64), (8192, 20), (8192, 64)])
 @pytest.mark.parametrize("ties", [False, True])
 def test_candidates_against_sort(q, ctx, vocab, k, ties):
