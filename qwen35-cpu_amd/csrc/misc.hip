@@ -73,6 +73,12 @@ __global__ void l2_normalize_kernel(float *x, int width, float eps, float scale)
 // walking every token through the ring in memory took 1250 us (0.08 TB/s),
 // this form 21.0 us (4.7 TB/s).
 constexpr int kConvRun = 8;
+// Kernels other than 4 re-read their taps token by token, so a run takes as
+// long as walking about 12 tokens through the ring. Runs against the walk:
+// kernel 5 over 1000 channels 9.6 against 7.7 us at 8 tokens, 9.7 against 10.2
+// at 12, 9.7 against 12.8 at 16; kernel 9 over 6144 channels 13.8 against 10.1,
+// 14.3 and 18.4; over 64 channels they meet at 13. Below this the walk is taken.
+constexpr int kConvGeneralMin = 13;
 
 template <int V>
 struct ConvVec {
@@ -156,7 +162,8 @@ __global__ void conv1d_silu_runs_kernel(float *state, int ring, const float *inp
 
 // The same with one thread per channel walking the tokens in order through
 // the ring: for outputs that overlap the inputs (each token's input is read
-// before its output is written) and for kernels longer than a run.
+// before its output is written), for kernels longer than a run, and for the
+// few tokens where runs of a general kernel size are slower.
 __global__ void conv1d_silu_kernel(float *state, int ring, const float *input, long long stride, const float *w,
                                    float *out, int batch, int channels, int kernel, int begin, int end) {
   const int c = begin + static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
@@ -230,7 +237,7 @@ hipError_t launch_conv1d_silu(float *state, int ring, const float *input, long l
   const uintptr_t out1 = out0 + (static_cast<size_t>(batch - 1) * channels + end) * sizeof(float);
   const bool overlap = in0 < out1 && out0 < in1;
   const int runs = (batch + kConvRun - 1) / kConvRun;
-  if (overlap || kernel - 1 > kConvRun || runs > 65535) {
+  if (overlap || kernel - 1 > kConvRun || runs > 65535 || (kernel != 4 && batch < kConvGeneralMin)) {
     Q35_LAUNCH((conv1d_silu_kernel), (end - begin + 255) / 256, 256, 0, stream, state, ring, input, stride, w, out,
                batch, channels, kernel, begin, end);
     return hipGetLastError();

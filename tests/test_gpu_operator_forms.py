@@ -44,7 +44,7 @@ def test_conv1d_runs(q, ctx, orc, batch, ch, kern, begin, end, extra, in_place):
 
 
 @pytest.mark.parametrize("kern", [1, 2, 3, 4, 5, 9, 10])
-@pytest.mark.parametrize("batch,ch", [(1, 64), (7, 68), (40, 66), (130, 64)])
+@pytest.mark.parametrize("batch,ch", [(1, 64), (7, 68), (12, 64), (13, 64), (40, 66), (130, 64)])
 def test_conv1d_bits_do_not_depend_on_the_form(q, ctx, batch, ch, kern):
     """The sum of a token is one fma chain (its own tap's product, then the
     history oldest first) in every form: four channels per thread or one, taps
