@@ -145,51 +145,97 @@ __global__ __launch_bounds__(1024) void gemm_direct_kernel(DirectArgs a) {
 
 }  // namespace
 
-// LDS bytes of a workgroup's split sums; launches keep within one 64 KiB window.
+// LDS bytes of a workgroup's split sums (at most 32 splits); launches keep
+// within one 64 KiB window.
 constexpr size_t kDirectMaxLds = 64 * 1024;
 static size_t direct_lds(int splits, int nt) { return static_cast<size_t>(splits) * nt * 1024; }
 
-// The line between this kernel and the dense GEMM (layout + dense launch): the
-// dense tiles do less work per output but take a fixed time while they leave
-// compute units idle. Measured, 64-row x 32-token units over two per compute
-// unit: at 0.12 (1024 x 3584, 128 vectors) 10.3 against 38.0 us; at 0.5 (4096
-// x 2560, 128) 14.3 against 28.2; at 0.88 (4096 x 2560, 200) 25.1 against 28.7;
-// at 1.01 (8224 x 2560, 128) 32.1 against 28.8; at 2.0 (4096 x 2560, 512) 52.8
-// against 31.3. Up to 64 vectors it beats the split launches at every shape
-// tried (18432 x 2560: 20 vectors 18.8 against 20.8, 64 vectors 32.3 against 39.0).
-bool gemm_direct_fits(int rows, int nb, size_t tokens, int cu_count) {
+struct DirectShape {
+  int splits, nt, groups, tiles;  // token tiles per workgroup; workgroups over rows and tokens
+};
+static DirectShape direct_shape(int rows, int nb, int tokens, int cus) {
+  DirectShape d;
+  d.splits = gemm_dense_splits(rows, nb, cus, 0);
+  d.groups = (rows + 15) / 16;
+  // token tiles per workgroup: as few as keep the launch within 14 wavefronts
+  // per compute unit, where a workgroup's own latency sets the time (1024 x
+  // 3584, 64 vectors: 5.4 us with one tile, 10.2 with four); beyond that more
+  // tiles share each weight load and unpack (18432 x 2560, 64 vectors: 44.0 us
+  // with one tile, 32.1 with four)
+  const int waves = std::min(d.splits, 16);
+  d.nt = 1;
+  while (d.nt < 4 && 16 * d.nt < tokens &&
+         static_cast<long long>(d.groups) * ((tokens + 16 * d.nt - 1) / (16 * d.nt)) * waves > 14LL * cus)
+    d.nt <<= 1;
+  while (d.nt > 1 && direct_lds(d.splits, d.nt) > kDirectMaxLds) d.nt >>= 1;
+  d.tiles = (tokens + 16 * d.nt - 1) / (16 * d.nt);
+  return d;
+}
+
+// The lines between this kernel, the split launches (up to 64 vectors) and the
+// dense GEMM (more), measured over 8 to 65536 rows and 8 to 512 blocks. Counted
+// in `per_cu`, the token rows that the busiest compute unit takes in all, and
+// the blocks of each.
+//
+// X4, up to 64 vectors: direct, 1.1 to 2.8 times as fast (18432 x 2560: 20
+// vectors 18.9 against 20.8 us, 64 vectors 32.2 against 38.4), except for work
+// above 20480 blocks per unit where
+//   - 33 to 48 vectors leave a quarter or more of four-tile workgroups empty
+//     (8224 x 128 blocks, 40 vectors: 27.5 against 24.2 us; 18432 x 160: 57.3
+//     against 52.3; below, 8224 x 96: 19.6 against 20.6). From 257 to 288 blocks
+//     the split launch's 32 partial rows cost as much (18432 x 288: 96.9
+//     against 105.3);
+//   - more than 352 blocks meet the two tiles that 32 splits leave room for
+//     (8224 x 512, 20 vectors: 57.3 against 44.9; 8224 x 352: 40.3 against 42.3).
+// X4, more vectors: direct where the dense tiles would leave compute units idle
+// (4096 x 80 blocks, 200 vectors: 24.6 against 29.0 us), up to 256 token rows
+// per unit, beyond for at most 64 blocks (320 rows: 8224 x 64, 96 vectors 22.9
+// against 24.1, 8224 x 112 42.6 against 38.4).
+// X1: a token's blocks lie 40 bytes apart in rows of their own, so a lane's
+// loads share no cache line with its neighbours' and each block of a token
+// costs a compute unit about 3.8 ns. Up to 64 vectors that has to stay below
+// the two launches saved: 2000 blocks per unit, a workgroup counted as 64 more
+// (8224 x 32 blocks, 7 vectors, 864: 6.3 against 11.2 us; 8224 x 64, 8 vectors,
+// 1728: 10.9 against 11.6; 18432 x 80, 5 vectors, 2320: 19.4 against 16.0; 32768
+// x 80, 64 vectors: 168 against 62). More vectors, against the dense GEMM's walk
+// of all blocks in one wavefront: 80 token rows per unit (1024 x 80 blocks, 67
+// vectors, 32 rows: 9.9 against 28.4; 2560 x 80, 96 vectors, 128 rows: 32.0
+// against 28.5).
+bool gemm_direct_fits(int rows, int nb, size_t tokens, int cu_count, bool x4) {
   if (tokens == 0 || tokens > size_t{65535} * 16) return false;  // grid.y
-  if (direct_lds(gemm_dense_splits(rows, nb, cu_count, 0), 1) > kDirectMaxLds) return false;
-  return tokens <= static_cast<size_t>(kMaxTokens) || !gemm_dense_fits(rows, static_cast<int>(tokens), cu_count);
+  const int n = static_cast<int>(tokens), cus = cu_count > 0 ? cu_count : 256;
+  const bool few = n <= kMaxTokens;
+  if (!few && gemm_dense_fits(rows, n, cus)) return false;
+  const DirectShape d = direct_shape(rows, nb, n, cus);
+  const long long rounds = (static_cast<long long>(d.groups) * d.tiles + cus - 1) / cus;
+  if (x4) {
+    const long long per_cu = rounds * 16 * d.nt;
+    if (!few) return per_cu <= 256 || nb <= 64;
+    const bool padded = n > 32 && n <= 48;
+    return per_cu * nb <= 20480 || n <= 16 || (padded ? nb > 256 && nb <= 288 : nb <= 352);
+  }
+  const long long per_wg = std::min(16 * d.nt, n);
+  return few ? rounds * (per_wg * nb + 64) <= 2000 : rounds * per_wg <= 80;
 }
 
 hipError_t launch_gemm_direct(const q35_q4_0_block_x8 *w, const void *act, bool x4, int rows, int nb, int tokens,
                               float *out, long long stride, int cu_count, hipStream_t stream) {
-  if (!gemm_direct_fits(rows, nb, tokens, cu_count) || (x4 && tokens % 4 != 0) || stride < rows)
+  if (!gemm_direct_fits(rows, nb, tokens, cu_count, x4) || (x4 && tokens % 4 != 0) || stride < rows)
     return hipErrorInvalidValue;
+  const DirectShape d = direct_shape(rows, nb, tokens, cu_count > 0 ? cu_count : 256);
   DirectArgs a;
   a.w = reinterpret_cast<const uint8_t *>(w);
   a.act = static_cast<const uint8_t *>(act);
   a.rows = rows;
   a.nb = nb;
   a.tokens = tokens;
-  a.splits = gemm_dense_splits(rows, nb, cu_count, 0);
+  a.splits = d.splits;
   a.out = out;
   a.stride = stride;
   a.vec_out = stride % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-  // token tiles per workgroup: as few as keep the launch within 14 wavefronts
-  // per compute unit, where a workgroup's own latency sets the time (1024 x
-  // 3584, 64 vectors: 5.4 us with one tile, 10.2 with four); beyond that more
-  // tiles share each weight load and unpack (18432 x 2560, 64 vectors: 44.0 us
-  // with one tile, 32.1 with four)
-  const int waves = std::min(a.splits, 16), groups = (rows + 15) / 16, cus = cu_count > 0 ? cu_count : 256;
-  int nt = 1;
-  while (nt < 4 && 16 * nt < tokens &&
-         static_cast<long long>(groups) * ((tokens + 16 * nt - 1) / (16 * nt)) * waves > 14LL * cus)
-    nt <<= 1;
-  while (nt > 1 && direct_lds(a.splits, nt) > kDirectMaxLds) nt >>= 1;
-  const dim3 grid(groups, (tokens + 16 * nt - 1) / (16 * nt)), block(64 * waves);
-  const size_t lds = direct_lds(a.splits, nt);
+  const int nt = d.nt;
+  const dim3 grid(d.groups, d.tiles), block(64 * std::min(d.splits, 16));
+  const size_t lds = direct_lds(d.splits, nt);
 #define Q35_DIRECT(NT, KS)                                                                             \
   if (x4)                                                                                              \
     Q35_LAUNCH((gemm_direct_kernel<true, NT, KS>), grid, block, lds, stream, a);                    \

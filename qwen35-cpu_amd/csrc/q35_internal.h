@@ -301,10 +301,9 @@ hipError_t launch_dot4_matvec(const q35_q4_0_block_x8 *w, const void *act, bool 
 bool gemm_dense_fits(int rows, int tokens, int cu_count);
 
 // The contraction of the split launches in one launch over X4 (tokens % 4 ==
-// 0) or X1 activations, without scratch: where gemm_direct_fits says so (one
-// split launch's tokens, or more where the dense GEMM would leave compute
-// units idle).
-bool gemm_direct_fits(int rows, int nb, size_t tokens, int cu_count);
+// 0) or X1 activations, without scratch: where gemm_direct_fits says that it is
+// the faster form.
+bool gemm_direct_fits(int rows, int nb, size_t tokens, int cu_count, bool x4);
 hipError_t launch_gemm_direct(const q35_q4_0_block_x8 *w, const void *act, bool x4, int rows, int nb, int tokens,
                               float *out, long long stride, int cu_count, hipStream_t stream);
 // Tokens per launch of the kernel-level dense path.

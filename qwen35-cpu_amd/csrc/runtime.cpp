@@ -278,7 +278,8 @@ size_t dot4_matmul_scratch_bytes(int rows, int nb, int chunk, bool argmax, int c
 static bool dot4_matmul_direct(const Context *ctx, const q35_q4_0_block_x8 *m, const q35_q8_0_block_x4 *x4,
                                const q35_q8_0_block_x1 *x1, const float *out, size_t rows, size_t vectors,
                                size_t blocks, size_t stride) {
-  if (!gemm_direct_fits(static_cast<int>(rows), static_cast<int>(blocks), vectors, ctx->cu_count)) return false;
+  if (!gemm_direct_fits(static_cast<int>(rows), static_cast<int>(blocks), vectors, ctx->cu_count, x4 != nullptr))
+    return false;
   const uintptr_t o0 = reinterpret_cast<uintptr_t>(out), o1 = o0 + ((vectors - 1) * stride + rows) * sizeof(float);
   const auto apart = [&](const void *p, size_t bytes) {
     const uintptr_t p0 = reinterpret_cast<uintptr_t>(p);

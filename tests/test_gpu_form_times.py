@@ -1,0 +1,36 @@
+"""Forms of one operator whose dispatch chooses the faster: the chosen one is
+timed against a call that the other form takes, or that does the same work in
+another layout. Bounds lie well above the run to run spread (about 3%)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _us(q, ctx, call, calls=50):
+    """Best of five rounds of `calls` calls, by the context's event timer."""
+    for _ in range(10):
+        call()
+    best = np.inf
+    for _ in range(5):
+        ctx.timer_begin()
+        for _ in range(calls):
+            call()
+        best = min(best, ctx.timer_end() * 1e3 / calls)
+    return best
+
+
+@pytest.mark.parametrize("rows,blocks,tokens", [(32768, 80, 64), (18432, 80, 16), (2560, 80, 256)])
+def test_x1_rows_cost_about_what_x4_rows_do(q, ctx, rows, blocks, tokens):
+    """X1 rows lie apart in memory: reading them in place took 3.1, 2.1 and 3.0
+    times as long as X4 rows at these sizes; through the layout launch it is
+    1.1 to 1.6 times."""
+    rng = np.random.default_rng(0)
+    dm = ctx.array(rng.integers(0, 60, size=(rows // 8, blocks, 144), dtype=np.uint8))
+    x1 = ctx.array(np.zeros((tokens, blocks, 40), np.uint8))
+    x4 = ctx.array(np.zeros((tokens // 4, blocks, 152), np.uint8))
+    out = ctx.array(shape=(tokens, rows), dtype=np.float32)
+    print(f"X1 against X4 {rows} rows {blocks} blocks {tokens} tokens", flush=True)
+    t1 = _us(q, ctx, lambda: q.q4_dot4_matmul_x1(ctx, dm, x1, out, rows, tokens, blocks, rows))
+    t4 = _us(q, ctx, lambda: q.q4_dot4_matmul(ctx, dm, x4, out, rows, tokens, blocks, rows))
+    assert t1 < 1.85 * t4, (t1, t4)

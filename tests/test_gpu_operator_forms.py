@@ -189,6 +189,40 @@ def test_outputs_over_activations(q, ctx, orc, rows, blocks, tokens, x1, offset)
             np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
 
+@pytest.mark.parametrize("rows,blocks,tokens", [
+    (4096, 121, 16), (4096, 122, 16), (4104, 30, 20), (24, 31, 36),  # X1 direct or split (2000 blocks a unit)
+    (1024, 8, 420), (1024, 8, 900), (2560, 4, 160),                  # X1 direct or dense (80 rows a unit)
+    (8224, 64, 68), (8224, 65, 68), (4096, 80, 200),                 # X4 direct or dense (256 rows, 64 blocks)
+    (8224, 106, 40), (8224, 107, 40), (8224, 257, 36), (2560, 352, 64), (2560, 353, 64)])  # X4 direct or split
+def test_forms_on_both_sides_of_the_lines(q, ctx, orc, rows, blocks, tokens):
+    """One set of codes through every form that takes it: X1 and X4 outputs in
+    buffers of their own (the direct GEMM, or the split launches or the dense
+    GEMM beyond its lines) and over their activations (never direct) have the
+    same bits."""
+    rng = np.random.default_rng(rows + blocks + tokens)
+    dm = ctx.array(orc.dot4_pack(orc.random_q4_blocks(rng, rows, 32 * blocks), rows, blocks))
+    codes = rng.integers(-127, 128, size=(tokens, blocks, 32)).astype(np.int8)
+    scales = rng.uniform(0.001, 0.02, size=(tokens, blocks)).astype(np.float32)
+    x1 = np.zeros((tokens, blocks), np.dtype([("s", "<f4"), ("sum", "<i2"), ("q", "i1", 32), ("pad", "<i2")]))
+    x1["s"], x1["sum"], x1["q"] = scales, codes.sum(-1), codes
+    x4 = np.zeros((tokens // 4, blocks), np.dtype([("s", "<f4", 4), ("sum", "<i2", 4), ("q", "i1", (4, 32))]))
+    x4["s"] = scales.reshape(-1, 4, blocks).transpose(0, 2, 1)
+    x4["q"] = codes.reshape(-1, 4, blocks, 32).transpose(0, 2, 1, 3)
+    x4["sum"] = x4["q"].sum(-1)
+    print(f"forms {rows} rows {blocks} blocks {tokens} tokens", flush=True)
+    want = None
+    for call, act in ((q.q4_dot4_matmul, x4), (q.q4_dot4_matmul_x1, x1)):
+        act = act.view(np.uint8).ravel()
+        apart = ctx.array(shape=(tokens, rows), dtype=np.float32)
+        call(ctx, dm, ctx.array(act), apart, rows, tokens, blocks, rows)
+        both = ctx.array(np.concatenate([act, np.zeros(max(0, tokens * rows * 4 - act.size), np.uint8)]))
+        call(ctx, dm, both, both, rows, tokens, blocks, rows)
+        over = both.download()[:tokens * rows * 4].view(np.uint32).reshape(tokens, rows)
+        want = over if want is None else want
+        np.testing.assert_array_equal(apart.download().view(np.uint32), want)
+        np.testing.assert_array_equal(over, want)
+
+
 @pytest.mark.parametrize("blocks", [1, 31, 32, 33, 64, 65, 97, 128, 129, 257, 288, 289, 577])
 def test_gemv_passes(q, ctx, orc, blocks):
     """Every step count and pass boundary of the GEMV, one to four vectors:
