@@ -375,12 +375,17 @@ constexpr size_t kHeadMaxLds = 64 * 1024;
 // accumulators of more token tiles need more registers
 constexpr int head_waves_per_simd(int nt) { return nt == 1 ? 3 : 2; }
 
+// How the greedy head applies the repetition penalty: not at all (no token of
+// the launch has one), with the counts read at the end of a row group, or with
+// the counts read ahead in the weight ring.
+enum HeadCounts { kCountsNone, kCountsAtEnd, kCountsAhead };
+
 template <int KS, bool G16>
 struct HeadChunk {
   q35_u32x4 q[KS];
   q35_u32x2 d[KS];
   q35_u32x2 d2[G16 ? KS : 1];  // G16: the scales of columns 16-31
-  q35_u32x4 n;                 // one token tile with penalties: counts of four rows of one token
+  q35_u32x4 n;                 // kCountsAhead: counts of four rows of one token
 };
 
 // Four adjacent occurrence counts (any int32 alignment).
@@ -403,10 +408,12 @@ __device__ __forceinline__ unsigned counted_rows(q35_u32x4 n) {
 // per block as half 0 then half 1, acc = fma(float(dot), d_half * s, acc)
 // (q4_g16_matmul_wide, q4_g16_evex.cpp:25-49). G16 launches use a two-chunk
 // ring: with three, the second scale words spill at the head's occupancy.
-template <int KS, int R, int NT, bool ARGMAX, int OCC, bool G16>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void head_kernel(GemmArgs a,
-                                                                                               int gpw) {
+template <int KS, int R, int NT, bool ARGMAX, bool G16, HeadCounts COUNTS>
+__device__ __forceinline__ void head_body(const GemmArgs &a, int gpw) {
   static_assert(R >= 2, "the ring loads the next chunk before computing the current one");
+  static_assert(COUNTS == kCountsNone || ARGMAX, "logits take no penalty here");
+  static_assert(COUNTS != kCountsAhead || NT == 1, "counts ahead: one token tile");
+  using Chunk = HeadChunk<KS, G16>;
   Q35_DYNAMIC_SHARED(uint64_t, lcodes);  // [NT][nb][64] A16 words, then float [NT][nb][16]
   const int nb = a.nb;
   float *lscales = reinterpret_cast<float *>(lcodes + static_cast<size_t>(NT) * nb * 64);
@@ -421,24 +428,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   constexpr int kTile = G16 ? 160 : 144, kCodes = G16 ? 32 : 16;
   const size_t tile_bytes = static_cast<size_t>(nb) * kTile;
 
-  // Occurrence counts of the repetition penalty. With one token tile they
-  // travel in the ring: chunk i < 4 of a group also loads the lane's four rows'
-  // counts of its token 4G + i (later chunks, whose loads stay unconditional,
-  // a word of the codes), so a group of four or more chunks has them all
-  // before its epilogue. Read there, each token's counts were a round trip
-  // that drained the ring. More tiles read them in the epilogue, a tile's at
-  // once. A call of 248320 x 1024: 16 tokens 48.6 -> 44.6 us, 32 tokens 70.9
-  // -> 55.7.
-  constexpr bool kCountsAhead = ARGMAX && NT == 1;
-  const bool ahead = kCountsAhead && cpg >= 4;
-  const int32_t *unused = reinterpret_cast<const int32_t *>(a.codes);  // a readable place
-  const int32_t *cbase[4] = {unused, unused, unused, unused};
+  // Counts ahead: chunk i < 4 of a group also loads the lane's four rows'
+  // counts of its token 4G + i (later chunks, and tokens without a penalty,
+  // whose loads stay unconditional, the first word of the counts), so a group
+  // of four or more chunks has them all before its epilogue. Read there, each
+  // token's counts were a round trip that drained the ring.
   unsigned seen = 0;  // bit 4j + r: row r of token 4G + j in the group being computed
+  // per-token penalty and counts row (loop invariant; loaded before the
+  // weights so that the group epilogues never wait on a load)
+  float pen[NT][4];
+  int crow[NT][4];  // kCountsAhead: -1 for a token without a penalty
+  if constexpr (COUNTS != kCountsNone) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int tok = min(t * 16 + 4 * G + j, a.tokens - 1);
+        pen[t][j] = a.penalties[tok];
+        crow[t][j] = a.count_rows != nullptr ? a.count_rows[tok] : tok;
+        if (COUNTS == kCountsAhead && !(pen[t][j] > 1.0F)) crow[t][j] = -1;
+      }
+  }
 
   // next chunk to load: group lg, chunk lch (advanced after every load);
   // past the last chunk the last one is loaded again
   int lg = g0, lch = 0;
-  auto load = [&](HeadChunk<KS, G16> &buf) {
+  auto load = [&](Chunk &buf) {
     const bool past = lg >= g1;
     const int gl = max(past ? g1 - 1 : lg, 0), cl = past ? cpg - 1 : lch;
     const int rt = min(gl * 8 + T, ntiles - 1);
@@ -450,10 +465,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
       buf.d[i] = *reinterpret_cast<const q35_u32x2 *>(tile + b * kTile + 8 * h);
       if constexpr (G16) buf.d2[i] = *reinterpret_cast<const q35_u32x2 *>(tile + b * kTile + 16 + 8 * h);
     }
-    if constexpr (kCountsAhead) {
-      const int32_t *p01 = (cl & 1) ? cbase[1] : cbase[0], *p23 = (cl & 1) ? cbase[3] : cbase[2];
-      const int32_t *p = cl >= 4 ? unused : (cl & 2) ? p23 : p01;
-      buf.n = load_counts(p == unused ? p : p + min(gl * kRowsPerGroup + 4 * c, a.rows - 4));
+    if constexpr (COUNTS == kCountsAhead) {
+      const int r01 = (cl & 1) ? crow[0][1] : crow[0][0], r23 = (cl & 1) ? crow[0][3] : crow[0][2];
+      const int r = cl >= 4 ? -1 : (cl & 2) ? r23 : r01;
+      const long long at = static_cast<long long>(r) * a.counts_stride + min(gl * kRowsPerGroup + 4 * c, a.rows - 4);
+      buf.n = load_counts(a.counts + (r < 0 ? 0 : at));
     }
     if (++lch == cpg) {
       lch = 0;
@@ -461,26 +477,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     }
   };
 
-  // per-token penalty and counts row (loop invariant; loaded before the
-  // weights so that the group epilogues never wait on a load)
-  float pen[NT][4];
-  int crow[NT][4];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int tok = min(t * 16 + 4 * G + j, a.tokens - 1);
-      pen[t][j] = ARGMAX && a.penalties != nullptr ? a.penalties[tok] : 1.0F;
-      crow[t][j] = ARGMAX && a.count_rows != nullptr ? a.count_rows[tok] : tok;
-    }
-  if constexpr (kCountsAhead) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (a.counts != nullptr && pen[0][j] > 1.0F)
-        cbase[j] = a.counts + static_cast<long long>(crow[0][j]) * a.counts_stride;
-  }
-
-  HeadChunk<KS, G16> buf[R];
+  Chunk buf[R];
   load(buf[0]);
   // stage the activations; the first pass is issued before chunks 1..R-2, so
   // waiting for it leaves those chunks in flight
@@ -521,11 +518,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[t][i][j] = 0.0F;
-  unsigned long long run_best[NT][4];
+  unsigned long long run_best[NT];  // of token 16t + 4G + c % 4
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) run_best[t][j] = 0ull;
+  for (int t = 0; t < NT; ++t) run_best[t] = 0ull;
   const bool vec_out = (a.stride & 3) == 0;
 
   // group cg, chunk cch of the next compute
@@ -534,12 +529,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     const int row0 = cg * kRowsPerGroup + 4 * c;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      if (ARGMAX && !ahead) {
+      if constexpr (COUNTS == kCountsAtEnd) {
         q35_u32x4 n[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           n[j] = q35_u32x4{0u, 0u, 0u, 0u};
-          if (pen[t][j] > 1.0F && a.counts != nullptr && row0 < a.rows)
+          if (pen[t][j] > 1.0F && row0 < a.rows)
             n[j] = load_counts(a.counts + static_cast<long long>(crow[t][j]) * a.counts_stride + row0);
         }
         seen = 0;
@@ -552,14 +547,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
         if constexpr (ARGMAX) {
           unsigned long long key = 0ull;
           if (tok < a.tokens) {
-            const float p = pen[t][j];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int row = row0 + r;
               if (row >= a.rows) continue;
               float val = acc[t][r][j];
-              if (p > 1.0F && a.counts != nullptr && ((seen >> (4 * j + r)) & 1u) != 0u)
-                val = val > 0.0F ? val / p : val * p;
+              if constexpr (COUNTS != kCountsNone) {
+                const float p = pen[t][j];
+                if (p > 1.0F && ((seen >> (4 * j + r)) & 1u) != 0u) val = val > 0.0F ? val / p : val * p;
+              }
               const unsigned long long k = argmax_key(val, static_cast<uint32_t>(row));
               key = k > key ? k : key;
             }
@@ -569,7 +565,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
             const unsigned long long o = __shfl_xor(key, m, 64);
             key = o > key ? o : key;
           }
-          run_best[t][j] = key > run_best[t][j] ? key : run_best[t][j];
+          // every lane of the 16 now has the token's key: one of them keeps it
+          if ((c & 3) == j && key > run_best[t]) run_best[t] = key;
         } else {
           if (tok < a.tokens && row0 < a.rows)
             store_row4(a.out + static_cast<size_t>(tok) * a.stride + row0, vec_out, acc[t][0][j], acc[t][1][j],
@@ -581,8 +578,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
     }
     seen = 0;
   };
-  auto compute = [&](HeadChunk<KS, G16> &cur) {
-    if constexpr (kCountsAhead) seen |= cch < 4 ? counted_rows(cur.n) << (4 * cch) : 0u;
+  auto compute = [&](Chunk &cur) {
+    if constexpr (COUNTS == kCountsAhead) seen |= cch < 4 ? counted_rows(cur.n) << (4 * cch) : 0u;
 #pragma unroll
     for (int i = 0; i < KS; ++i) {
       const int b = cch * KS + i;
@@ -659,16 +656,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC)))
   }
 
   if constexpr (ARGMAX) {
-    if (c == 0) {
+    if (c < 4) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int tok = t * 16 + 4 * G + j;
-          if (tok < a.tokens) a.cand[static_cast<size_t>(gw) * a.cand_stride + tok] = run_best[t][j];
-        }
+      for (int t = 0; t < NT; ++t) {
+        const int tok = t * 16 + 4 * G + c;
+        if (tok < a.tokens) a.cand[static_cast<size_t>(gw) * a.cand_stride + tok] = run_best[t];
+      }
     }
   }
+}
+
+template <int KS, int R, int NT, bool ARGMAX, int OCC, bool G16, HeadCounts COUNTS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) void head_kernel(GemmArgs a,
+                                                                                               int gpw) {
+  if constexpr (COUNTS != kCountsNone) {
+    // penalties that are all 1 (device values): the form without counts, half
+    // a microsecond for the look at them (248320 x 1024, 16 tokens: 34.5 us)
+    if (q35_ballot(a.penalties[min(static_cast<int>(threadIdx.x & 63), a.tokens - 1)] > 1.0F) == 0ull) {
+      head_body<KS, R, NT, ARGMAX, G16, kCountsNone>(a, gpw);
+      return;
+    }
+  }
+  head_body<KS, R, NT, ARGMAX, G16, COUNTS>(a, gpw);
 }
 
 // One workgroup per token: the best key over all workgroups' candidates,
@@ -854,19 +863,33 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream) {
     }
     if (hp.use) {
       const dim3 grid(hp.grid), block(64 * kHeadWaves);
-#define Q35_HEAD_G(NT, G16)                                                                                     \
-  if (argmax) {                                                                                                 \
-    Q35_LAUNCH((head_kernel<kHeadKS, (G16 ? 2 : kHeadRing), NT, true, head_waves_per_simd(NT), G16>), grid, block, hp.smem,  \
-               stream, a, hp.gpw);                                                                              \
-  } else {                                                                                                      \
-    Q35_LAUNCH((head_kernel<kHeadKS, (G16 ? 2 : kHeadRing), NT, false, head_waves_per_simd(NT), G16>), grid, block, hp.smem, \
-               stream, a, hp.gpw);                                                                              \
-  }
+      // Without counts or penalties: the form without them (248320 x 1024, 16
+      // tokens: 34.1 us a call; a form that always carries counts in the ring
+      // spilled registers and took 38.3). With them, one token tile whose
+      // wavefronts walk several groups of four or more chunks reads them ahead
+      // (39.2 us; at the groups' ends, token by token, 42.2). A wavefront of one
+      // group has nothing left in its ring to drain and reads them at the end
+      // (60000 x 2048, 16 tokens: 26.5 us, ahead 28.1), as several tiles do, whose
+      // registers hold no more (32 tokens: 52.6 us, token by token 62.0).
+      const bool counted = argmax && a.counts != nullptr && a.penalties != nullptr;
+      const bool ahead = (a.nb + kHeadKS - 1) / kHeadKS >= 4 && hp.gpw > 1;
+#define Q35_HEAD_G(NT, ARGMAX, G16, COUNTS)                                                                         \
+  Q35_LAUNCH((head_kernel<kHeadKS, (G16 ? 2 : kHeadRing), NT, ARGMAX, head_waves_per_simd(NT), G16, COUNTS>), grid, \
+             block, hp.smem, stream, a, hp.gpw)
+#define Q35_HEAD_C(NT, G16)                          \
+  if (!argmax)                                       \
+    Q35_HEAD_G(NT, false, G16, kCountsNone);         \
+  else if (!counted)                                 \
+    Q35_HEAD_G(NT, true, G16, kCountsNone);          \
+  else if (NT == 1 && ahead)                         \
+    Q35_HEAD_G(1, true, G16, kCountsAhead);          \
+  else                                               \
+    Q35_HEAD_G(NT, true, G16, kCountsAtEnd);
 #define Q35_HEAD(NT)         \
   if (a.g16) {               \
-    Q35_HEAD_G(NT, true)     \
+    Q35_HEAD_C(NT, true)     \
   } else {                   \
-    Q35_HEAD_G(NT, false)    \
+    Q35_HEAD_C(NT, false)    \
   }
       switch (hp.nt) {
         case 1: Q35_HEAD(1) break;
@@ -875,6 +898,7 @@ hipError_t launch_gemm(const GemmArgs &a, hipStream_t stream) {
         default: Q35_HEAD(4) break;
       }
 #undef Q35_HEAD
+#undef Q35_HEAD_C
 #undef Q35_HEAD_G
       return hipGetLastError();
     }

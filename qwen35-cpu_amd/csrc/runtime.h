@@ -40,8 +40,9 @@ struct StepShape {
   int attn_rows = 0;           // rows of one-row segments (the decode attention kernel in a packed step)
   bool single = true;          // every segment is one row (the decode kernels)
   bool heads_identity = true;  // head h is row h
+  bool penalized = false;      // some head row has a penalty above 1 (the greedy head then reads counts)
   std::array<int, 8> key(bool want_logits) const {
-    return {rows, segments, heads, tiles, grid_splits, (single ? 1 : 0) | (heads_identity ? 2 : 0),
+    return {rows, segments, heads, tiles, grid_splits, (single ? 1 : 0) | (heads_identity ? 2 : 0) | (penalized && !want_logits ? 4 : 0),
             want_logits ? 1 : 0, attn_rows};
   }
 };

@@ -674,8 +674,10 @@ bool launch_events(hipEvent_t *start, hipEvent_t *stop) {
 // rt->meta_host; the host copy is part of the enqueued work so the whole
 // sequence can be captured as a graph.
 // The greedy head over `tokens` rows of A16 activations in rt->codes/scales:
-// penalty counts of slot count_rows[t], penalty penalties[t] (device arrays).
-static GemmArgs greedy_head_args(q35_runtime *rt, int tokens, const int32_t *count_rows, const float *penalties) {
+// penalty counts of slot count_rows[t], penalty penalties[t] (device arrays);
+// `penalized`: some penalty is above 1 (the head reads no counts otherwise).
+static GemmArgs greedy_head_args(q35_runtime *rt, int tokens, const int32_t *count_rows, const float *penalties,
+                                 bool penalized) {
   const q35_model_dims &d = rt->model->d;
   GemmArgs g;
   g.w = rt->model->embed;
@@ -687,7 +689,7 @@ static GemmArgs greedy_head_args(q35_runtime *rt, int tokens, const int32_t *cou
   g.tokens = tokens;
   g.cand = rt->cand;
   g.cand_stride = kMaxTokens;
-  g.counts = rt->counts;
+  g.counts = penalized ? rt->counts : nullptr;
   g.count_rows = count_rows;
   g.counts_stride = d.vocab;
   g.penalties = penalties;
@@ -1268,7 +1270,7 @@ int runtime_enqueue_step(q35_runtime *rt, const StepShape &sh, bool want_logits)
       Q35_KERNEL(Q35_KERNEL_HEAD, gemm_algorithmic_bytes(d.vocab, H / 32, n, true, false) + g16_extra,
                  launch_gemm(g, s), "logits head");
     } else {
-      GemmArgs g = greedy_head_args(rt, n, head_slots + h0, head_penalties + h0);
+      GemmArgs g = greedy_head_args(rt, n, head_slots + h0, head_penalties + h0, sh.penalized);
       g.codes = rt->codes + tile0 * (H / 32) * 64;
       g.scales = rt->scales + tile0 * (H / 32) * 16;
       const int ncand = gemm_argmax_cands(d.vocab, H / 32, n, ctx->cu_count, 0, m->embed_g16);
@@ -1373,6 +1375,7 @@ int pack_segments(q35_runtime *rt, const q35_segment *segs, int n, StepShape *sh
       head_rows[heads] = r - 1;
       head_slots[heads] = g.slot;
       head_pen[heads] = g.penalty;
+      sh.penalized = sh.penalized || g.penalty > 1.0F;
       sh.heads_identity = sh.heads_identity && heads == r - 1;
       ++heads;
     }
@@ -1927,7 +1930,8 @@ extern "C" int q35_runtime_head(q35_runtime *rt, int32_t slot, const float *hidd
   p.scales = rt->scales;
   Q35_HIP_TRY(ctx, launch_prep(p, s));
   const GemmArgs g = greedy_head_args(rt, 1, reinterpret_cast<const int32_t *>(rt->meta_dev + ml.head_slots),
-                                      reinterpret_cast<const float *>(rt->meta_dev + ml.head_penalties));
+                                      reinterpret_cast<const float *>(rt->meta_dev + ml.head_penalties),
+                                      penalty > 1.0F);
   Q35_HIP_TRY(ctx, launch_gemm(g, s));
   const int ncand = gemm_argmax_cands(d.vocab, d.hidden / 32, 1, ctx->cu_count, 0, rt->model->embed_g16);
   Q35_HIP_TRY(ctx, launch_argmax_finalize(rt->cand, ncand, kMaxTokens, 1, rt->tokens_out_dev, nullptr, s));

@@ -34,3 +34,18 @@ def test_x1_rows_cost_about_what_x4_rows_do(q, ctx, rows, blocks, tokens):
     t1 = _us(q, ctx, lambda: q.q4_dot4_matmul_x1(ctx, dm, x1, out, rows, tokens, blocks, rows))
     t4 = _us(q, ctx, lambda: q.q4_dot4_matmul(ctx, dm, x4, out, rows, tokens, blocks, rows))
     assert t1 < 1.85 * t4, (t1, t4)
+
+
+@pytest.mark.parametrize("kernel,tokens,channels", [(9, 8, 6144), (7, 6, 6144), (5, 8, 1000)])
+def test_few_tokens_of_a_general_convolution(q, ctx, kernel, tokens, channels):
+    """Few tokens of kernels other than 4 walk the ring, as an in-place call
+    always does; in runs of tokens they took 1.37, 1.31 and 1.24 times as long."""
+    rng = np.random.default_rng(0)
+    state = ctx.array(rng.standard_normal((kernel - 1, channels)).astype(np.float32))
+    x = ctx.array(rng.standard_normal((tokens, channels)).astype(np.float32))
+    w = ctx.array((0.1 * rng.standard_normal((kernel, channels))).astype(np.float32))
+    out = ctx.array(shape=(tokens, channels), dtype=np.float32)
+    print(f"conv kernel {kernel} {tokens} tokens of {channels} channels", flush=True)
+    apart = _us(q, ctx, lambda: q.causal_conv1d_silu_f32(ctx, state, 0, x, w, out, channels, kernel, batch=tokens))
+    place = _us(q, ctx, lambda: q.causal_conv1d_silu_f32(ctx, state, 0, x, w, x, channels, kernel, batch=tokens))
+    assert apart < 1.15 * place, (apart, place)

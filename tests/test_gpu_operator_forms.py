@@ -336,3 +336,34 @@ def test_head_counts_of_the_best_rows(q, ctx, orc, rows, blocks, vectors):
                            blocks, idx, val)
     np.testing.assert_array_equal(idx.download(), want)
     np.testing.assert_array_equal(val.download(), adj[np.arange(vectors), want])
+
+
+@pytest.mark.parametrize("g16", [False, True])
+@pytest.mark.parametrize("rows", [5, 20])
+def test_greedy_steps_with_and_without_penalties(q, ctx, rows, g16):
+    """Steps of one shape whose rows have no, some or only penalties, in turn
+    and with captured graphs: each gives the tokens that its logits and counts
+    give, so a step with a penalty never replays the graph without counts."""
+    from tests.model_util import build_small_model, small_dims, upload_model
+    d, _ = small_dims()
+    d = dict(d, hidden=1024, intermediate=512, n_layers=2)
+    sched = np.array([1, 0], np.uint8)
+    model = upload_model(q, ctx, d, sched, build_small_model(d, sched, seed=23, head_g16=g16))
+    rt = q.Runtime(model, max_slots=rows, max_batch=32, max_context=16, page_tokens=16, use_graphs=True)
+    rng = np.random.default_rng(rows)
+    # most of the vocabulary counted in every slot, so that a penalty moves most maxima
+    slots = [rt.slot_alloc(rng.permutation(d["vocab"])[d["vocab"] // 16:].astype(np.int32)) for _ in range(rows)]
+    table = np.array([[rt.page_alloc()] for _ in range(rows)], np.int32)
+    toks = rng.integers(0, d["vocab"], size=rows).astype(np.int32)
+    one, some, most = np.ones(rows, np.float32), np.ones(rows, np.float32), np.full(rows, 4.0, np.float32)
+    some[::3] = 4.0
+    print(f"greedy steps rows {rows} G16 {g16}", flush=True)
+    # position 0 again each time: the step reads the state it found the first time
+    want = {}
+    for name, pen in (("one", one), ("some", some), ("most", most)):
+        want[name] = rt.step(slots, [0] * rows, toks, table, penalties=pen, logits=True)[0]
+    assert np.any(want["one"] != want["some"]) and np.any(want["some"] != want["most"])
+    for name, pen in (("one", one), ("some", some), ("one", one), ("most", most), ("one", one), ("some", some)):
+        np.testing.assert_array_equal(rt.step(slots, [0] * rows, toks, table, penalties=pen), want[name])
+    rt.close()
+    model.close()
