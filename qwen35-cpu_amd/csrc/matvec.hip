@@ -113,8 +113,18 @@ __global__ __launch_bounds__(kMvThreads) void dot4_matvec_kernel(MvArgs a) {
     if (b0 + kPass < a.nb) load(b0 + kPass);
     if (tid < 8 * NV) {
       const int rr = tid & 7, v = tid >> 3;
-#pragma unroll 8
-      for (int bl = 0; bl < n; ++bl) {
+      int bl = 0;
+      for (; bl + 8 <= n; bl += 8) {
+        // eight reads, then their terms (without the fence the compiler reads
+        // and waits for one pair at a time: 1024 x 4096 4.65 against 3.7 us)
+        q35_f32x2 p[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[e] = fs[v][rr][bl + e];
+        q35_compiler_fence();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) res = fmaf(p[e][0], p[e][1], res);
+      }
+      for (; bl < n; ++bl) {
         const q35_f32x2 p = fs[v][rr][bl];
         res = fmaf(p[0], p[1], res);
       }
@@ -137,7 +147,11 @@ hipError_t launch_dot4_matvec(const q35_q4_0_block_x8 *w, const void *act, bool 
   a.out = out;
   a.stride = stride;
   const dim3 grid(rows / 8), block(kMvThreads);
-  // as many steps per pass as the row has blocks, up to four
+  // As many steps per pass as the row has blocks, up to four. Longer rows are
+  // passes of four: one pass of nine steps for one vector has 140 registers
+  // and repeats its last block where the row is shorter (18432 rows: 160 blocks
+  // 17.2 against 13.5 us, 288 blocks 23.1 against 22.6, 320 blocks 32.5 against
+  // 24.2; it is ahead only for 257 to 288 blocks of few rows, 1024: 6.3 against 6.6).
 #define Q35_MV(NV, X)                                                                                          \
   switch (std::min(4, (nb + kMvStep - 1) / kMvStep)) {                                                         \
     case 1: Q35_LAUNCH((dot4_matvec_kernel<NV, X, 1>), grid, block, 0, stream, a); break;                      \
@@ -149,15 +163,7 @@ hipError_t launch_dot4_matvec(const q35_q4_0_block_x8 *w, const void *act, bool 
     Q35_MV(4, true)
   } else {
     switch (count) {
-      case 1:
-        // rows past four steps in passes of up to nine (the 4B down projection's
-        // 288 blocks are one pass: 8.0 us against 10.5 in passes of four)
-        if (nb > 4 * kMvStep) {
-          Q35_LAUNCH((dot4_matvec_kernel<1, false, 9>), grid, block, 0, stream, a);
-        } else {
-          Q35_MV(1, false)
-        }
-        break;
+      case 1: Q35_MV(1, false) break;
       case 2: Q35_MV(2, false) break;
       case 3: Q35_MV(3, false) break;
       default: Q35_MV(4, false) break;

@@ -49,3 +49,19 @@ def test_few_tokens_of_a_general_convolution(q, ctx, kernel, tokens, channels):
     apart = _us(q, ctx, lambda: q.causal_conv1d_silu_f32(ctx, state, 0, x, w, out, channels, kernel, batch=tokens))
     place = _us(q, ctx, lambda: q.causal_conv1d_silu_f32(ctx, state, 0, x, w, x, channels, kernel, batch=tokens))
     assert apart < 1.15 * place, (apart, place)
+
+
+@pytest.mark.parametrize("rows,blocks", [(512, 128), (1024, 120)])
+def test_gemv_chain_reads_ahead(q, ctx, rows, blocks):
+    """Four steps of the one-vector GEMV against three: a third more blocks
+    took 1.25 times as long where the chain waited for every pair of terms
+    that it reads; reading eight at once it is about 1.05 times."""
+    rng = np.random.default_rng(0)
+    out = ctx.array(shape=(1, rows), dtype=np.float32)
+    us = {}
+    for nb in (96, blocks):
+        dm = ctx.array(rng.integers(0, 60, size=(rows // 8, nb, 144), dtype=np.uint8))
+        x1 = ctx.array(np.zeros((1, nb, 40), np.uint8))
+        print(f"GEMV {rows} rows {nb} blocks", flush=True)
+        us[nb] = _us(q, ctx, lambda: q.q4_dot4_matmul_x1(ctx, dm, x1, out, rows, 1, nb, rows), 400)
+    assert us[blocks] < 1.15 * us[96], us
