@@ -374,27 +374,32 @@ __global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_kernel(Attn
 // The same over exactly the chunks that rows row0 .. row0 + n - 1 have, where
 // the host knows their context lengths: first[i] is the number of chunks
 // before row i, so workgroup x finds its row by bisection (scalar loads of the
-// kernel arguments). A grid as wide as the longest context launches a
+// kernel arguments). The order is the full grid's, row by row and within a row
+// KV head by head (all rows of one head first: 200 rows of 2550 tokens, 4 KV
+// heads, 500 against 489 us). A grid as wide as the longest context launches a
 // workgroup for every chunk a shorter row lacks, which costs a dispatch and a
-// round trip before it returns (64 rows, contexts 128 to 8192: half of them;
-// 16 rows of 64 to 4096: 43.5 -> 35.0 us a call with the lengths read back
-// through pinned memory, 1 row of 8000: 38.0 -> 30.6).
-constexpr int kRaggedRows = 64;
+// round trip before it returns (200 rows of about 600 tokens and one of 2000, 4 KV
+// heads: 259.6 -> 137.0 us; 64 rows of 150 to 500: 42 -> 35). 256 rows per launch
+// keep the arguments near 1 KiB (0.1 to 0.3 us more than 64 rows' arguments); a
+// second launch costs about 5 us (65 rows of 62 to 500 tokens, 2 KV heads: 33.7 us
+// in groups of 64, 28.5 in one).
+constexpr int kRaggedRows = 256;
 struct RaggedRows {
-  int n, row0;
+  int n, row0;  // rows, the first of them
   int first[kRaggedRows + 1];
 };
 
 template <int QPK, bool GROUPS>
 __global__ __launch_bounds__(256) Q35_WAVES_PER_EU(2) void attention_ragged_kernel(AttnArgs a, RaggedRows rows) {
-  const int x = static_cast<int>(blockIdx.x);
+  const int x = static_cast<int>(blockIdx.x), kv = a.kv_heads;
   int lo = 0, hi = rows.n;  // first[lo] <= x < first[hi]
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
-    if (rows.first[mid] <= x) lo = mid;
+    if (rows.first[mid] * kv <= x) lo = mid;
     else hi = mid;
   }
-  attention_chunk<QPK, GROUPS>(a, x - rows.first[lo], static_cast<int>(blockIdx.y), rows.row0 + lo);
+  const int n = rows.first[lo + 1] - rows.first[lo], rem = x - rows.first[lo] * kv, g = rem / n;
+  attention_chunk<QPK, GROUPS>(a, rem - g * n, g, rows.row0 + lo);
 }
 
 // Prefill and packed steps: one workgroup per (tile of up to kAttnTileRows
@@ -834,19 +839,26 @@ hipError_t launch_attention(const AttnArgs &a, hipStream_t stream) {
   // tiled: the prompt tiles, then the one-row segments' rows as decode rows
   const int decode_rows = tiled ? a.row_count : a.batch;
   if (tiled && a.tiles > 0 && (a.prompt_o == nullptr || a.prompt_ml == nullptr)) return hipErrorInvalidValue;
-  // known context lengths: only the chunks that the rows have, unless that
-  // saves less than a tenth of the grid
+  // Known context lengths: only the chunks that the rows have, where that
+  // saves a tenth of the grid and enough workgroups: the bisection costs about
+  // 0.5 us and each launch after the first 5 us, an idle workgroup 2 to 3 ns (64
+  // rows of 2 KV heads, one of 3 chunks and the rest 2, 126 saved: 23.4 against
+  // 22.5 us for the full grid; 500 tokens of which 80%, 252 saved: 38.1 against
+  // 40.1; 400 rows, 3192 saved over two launches: 81.7 against 92.9; at 0.96 of
+  // the grid the two meet).
   long long chunks = 0;
   if (!tiled && a.row_list == nullptr && a.host_lens != nullptr)
     for (int r = 0; r < a.batch; ++r) chunks += (a.host_lens[r] + kChunkTokens - 1) / kChunkTokens;
-  const bool ragged = chunks > 0 && 10 * chunks < 9LL * gs * a.batch;
+  const long long full = static_cast<long long>(gs) * a.batch, launches = (a.batch + kRaggedRows - 1) / kRaggedRows;
+  const bool ragged =
+      chunks > 0 && 10 * chunks < 9 * full && (full - chunks) * a.kv_heads >= 128 + 2048 * (launches - 1);
 #define Q35_ATTN(Q)                                                                                    \
   if (tiled && a.tiles > 0)                                                                            \
     Q35_LAUNCH((attention_flash_kernel<Q>), dim3(a.tiles, a.kv_heads), dim3(128 * (Q)), 0, stream, a); \
   if (ragged) {                                                                                        \
     for (int row0 = 0; row0 < a.batch; row0 += kRaggedRows) {                                          \
       RaggedRows rows = ragged_rows(a, row0);                                                          \
-      const dim3 grid(rows.first[rows.n], a.kv_heads);                                                 \
+      const dim3 grid(rows.first[rows.n] * a.kv_heads);                                                 \
       if (a.page_tokens >= 8)                                                                          \
         Q35_LAUNCH((attention_ragged_kernel<Q, true>), grid, dim3(256), 0, stream, a, rows);           \
       else                                                                                             \

@@ -65,3 +65,28 @@ def test_gemv_chain_reads_ahead(q, ctx, rows, blocks):
         print(f"GEMV {rows} rows {nb} blocks", flush=True)
         us[nb] = _us(q, ctx, lambda: q.q4_dot4_matmul_x1(ctx, dm, x1, out, rows, 1, nb, rows), 400)
     assert us[blocks] < 1.15 * us[96], us
+
+
+def test_one_more_row_of_ragged_attention(q, ctx):
+    """65 rows of unequal contexts against 64: the one row took a launch of its
+    own and 1.22 times as long in groups of 64 rows; in one launch 1.03 times."""
+    rng = np.random.default_rng(5)
+    heads, kv, page = 8, 2, 16
+    us = {}
+    for rows in (64, 65):
+        lens = rng.integers(62, 501, size=rows).astype(np.int32)
+        lens[0] = 500
+        need = (lens + page - 1) // page
+        table = np.zeros((rows, need.max()), np.int32)
+        at = 0
+        for r in range(rows):
+            table[r, :need[r]] = np.arange(at, at + need[r])
+            at += need[r]
+        pool = ctx.array(np.zeros((at, page, kv, 256), np.uint16))
+        qv = ctx.array(np.zeros((rows, heads * 256), np.float32))
+        dt, dl = ctx.array(table), ctx.array(lens)
+        out = ctx.array(shape=(rows, heads * 256), dtype=np.float32)
+        print(f"attention {rows} rows", flush=True)
+        us[rows] = _us(q, ctx, lambda: q.attention_decode_paged(ctx, qv, qv, pool, pool, dt, table.shape[1], dl, page,
+                                                                out, rows, heads, kv, 256, 1.0 / 16.0))
+    assert us[65] < 1.12 * us[64], us

@@ -278,10 +278,12 @@ def test_x4_preparation_equals_rows(q, ctx, tokens, cols, h128):
 
 
 @pytest.mark.parametrize("batch,page_tokens,lens", [
-    (2, 16, (1, 700)), (3, 4, (130, 1, 64)), (64, 16, None), (65, 16, None), (130, 8, None)])
+    (2, 16, (1, 700)), (2, 16, (1, 7000)), (3, 4, (130, 1, 64)), (64, 16, None), (65, 16, None), (130, 8, None),
+    (256, 16, None), (257, 16, None)])
 def test_ragged_attention_equals_rows_alone(q, ctx, batch, page_tokens, lens):
     """Rows of unequal contexts in one call (the grid of exactly their chunks,
-    in groups of 64 rows) give the bits of each row called alone."""
+    in groups of 256 rows, or the full grid where that saves too little) give
+    the bits of each row called alone."""
     rng = np.random.default_rng(batch)
     heads, kv, hd = 4, 2, 256
     lens = np.asarray(lens if lens is not None else rng.integers(1, 500, size=batch), np.int32)
@@ -305,7 +307,7 @@ def test_ragged_attention_equals_rows_alone(q, ctx, batch, page_tokens, lens):
 
     print(f"ragged attention batch {batch} page {page_tokens}", flush=True)
     together = call(np.arange(batch))
-    for r in sorted({0, 1, batch // 2, min(63, batch - 1), min(64, batch - 1), batch - 1}):
+    for r in sorted({0, 1, batch // 2, min(63, batch - 1), min(64, batch - 1), min(255, batch - 1), batch - 1}):
         np.testing.assert_array_equal(call(np.array([r]))[0], together[r])
     with pytest.raises(q.Q35Error):
         lens[0] = table.shape[1] * page_tokens + 1
