@@ -50,11 +50,14 @@ int static_scratch_init(Context *ctx) {
 using namespace q35;
 
 // The same contraction and bits as q35_q4_dot4_matmul, with no device
-// allocation: tokens go through the GEMM in chunks of 64, 48, 32 or 16 (the
-// largest whose layout and partials fit the static array; the K split, and so
-// every output bit, does not depend on the chunk). Rejects shapes whose
-// 16-token chunk does not fit. Calls that overlap on one device race on the
-// array.
+// allocation: where the call's form needs scratch (not the GEMV's and not the
+// direct GEMM's), tokens go through the split launches in chunks of 64, 48, 32
+// or 16 (the largest whose layout and partials fit the static array; the K
+// split, and so every output bit, does not depend on the chunk). Shapes whose
+// 16-token chunk does not fit are rejected for more than four vectors whichever
+// form would run, so that what is accepted depends on the shape alone and not
+// on where the forms' lines lie. Callers treat calls that overlap in time on
+// one device as racing on the array.
 extern "C" int q35_q4_dot4_matmul_noalloc(q35_context *ctx, const q35_q4_0_block_x8 *matrix,
                                           const q35_q8_0_block_x4 *vectors, float *output, size_t rows,
                                           size_t vectors_count, size_t blocks, size_t stride) {
@@ -69,7 +72,7 @@ extern "C" int q35_q4_dot4_matmul_noalloc(q35_context *ctx, const q35_q4_0_block
     if (ctx->device >= 0 && ctx->device < kMaxDevices) ptr = g_static_ptr[ctx->device];
   }
   if (ptr == nullptr) return set_error(ctx, Q35_ERR_HIP, "static scratch not resolved for this device");
-  // one to four vectors run the single-launch GEMV, which needs no scratch
+  // (one to four vectors run the single-launch GEMV and have no limit)
   size_t chunk = vectors_count <= static_cast<size_t>(kMatvecMaxVectors) ? kMaxTokens : 0;
   for (size_t c = kMaxTokens; chunk == 0 && c >= 16; c -= 16) {
     if (dot4_matmul_scratch_bytes(static_cast<int>(rows), static_cast<int>(blocks), static_cast<int>(c), false,

@@ -6,6 +6,8 @@ relative (north-star bar 1e-3); argmax indices exact."""
 import numpy as np
 import pytest
 
+from tests.operand_util import copying_product
+
 pytestmark = pytest.mark.gpu
 
 
@@ -190,33 +192,35 @@ def test_argmax_head_shapes(q, ctx, orc, rows, cols, vectors):
 @pytest.mark.parametrize("rows,blocks,vectors", [(2560, 288, 300), (3584, 32, 512), (200, 112, 132), (1032, 80, 68),
                                                   (16392, 40, 100), (200, 8, 4136)])
 def test_dense_matches_split_launches(q, ctx, orc, rows, blocks, vectors):
-    """Above 64 vectors q4_dot4_matmul runs the dense GEMM (every K block of a
-    64-row group in one wavefront, the split structure folded in registers);
-    its rows must equal the 64-vector split launches bit for bit, here with
-    32, 4 and 14 K splits, a ragged row group and ragged token groups; 16392
-    rows give a tall matrix whose last 64-row group holds one 8-row tile.
-    4136 vectors are a 4096-vector chunk and a 40-vector one, which the dense
-    GEMM runs with one token tile per wavefront (its form at 64 rows)."""
+    """The dense GEMM (every K block of a 64-row group in one wavefront, the
+    split structure folded in registers), the 64-vector split launches and the
+    call's own form (the direct GEMM where it fits, else the dense one) give the
+    same bits, here with 32, 4, 14, 10, 5 and 1 K splits, a ragged row group and
+    ragged token groups; 16392 rows give a tall matrix whose last 64-row group
+    holds one 8-row tile. 4136 vectors are a 4096-vector chunk and a 40-vector
+    one, which the dense GEMM runs with one token tile per wavefront (its form
+    at 64 rows). The dense and split forms are reached by calls whose outputs
+    overlap their activations."""
     rng = np.random.default_rng(rows + vectors)
     packed, x = _problem(orc, rng, rows, blocks * 32, vectors)
     act = orc.h128_prepare_4(x)
     dm, da = ctx.array(packed), ctx.array(act)
     stride = rows + 4
-    dense = ctx.array(np.full((vectors, stride), -5.0, np.float32))
     print(f"dense rows={rows} blocks={blocks} vectors={vectors}", flush=True)
-    q.q4_dot4_matmul(ctx, dm, da, dense, rows, vectors, blocks, stride)
-    got = dense.download()
+    got = copying_product(ctx, q.q4_dot4_matmul, dm, act, rows, vectors, blocks, stride, -5.0)
     assert np.all(got[:, rows:] == -5.0)
+    plain = ctx.array(np.full((vectors, stride), -5.0, np.float32))
+    q.q4_dot4_matmul(ctx, dm, da, plain, rows, vectors, blocks, stride)
+    np.testing.assert_array_equal(plain.download().view(np.uint32), got.view(np.uint32))
     for t0 in range(0, vectors, 64):
         n = min(64, vectors - t0)
         # up to four vectors would run the GEMV's single chains: launch eight
         # (the group twice) and keep the first rows, which are batch-invariant
         sub = act[t0 // 4:(t0 + n) // 4]
         n_run = 8 if n <= 4 else n
-        part = ctx.array(shape=(n_run, stride), dtype=np.float32)
-        q.q4_dot4_matmul(ctx, dm, ctx.array(np.concatenate([sub, sub]) if n <= 4 else sub), part, rows, n_run,
-                         blocks, stride)
-        np.testing.assert_array_equal(got[t0:t0 + n, :rows].view(np.uint32), part.download()[:n, :rows].view(np.uint32),
+        part = copying_product(ctx, q.q4_dot4_matmul, dm, np.concatenate([sub, sub]) if n <= 4 else sub, rows, n_run,
+                               blocks, stride)
+        np.testing.assert_array_equal(got[t0:t0 + n, :rows].view(np.uint32), part[:n, :rows].view(np.uint32),
                                       err_msg=f"vectors {t0}..{t0 + n}")
     want = orc.dot4_matmul(packed, act, rows, vectors, blocks)
     assert np.max(np.abs(got[:, :rows] - want)) <= 1e-5 * np.abs(want).max()

@@ -8,6 +8,8 @@ rounding of one fp32 chain (2^-24 per term) unless exact."""
 import numpy as np
 import pytest
 
+from tests.operand_util import At
+
 pytestmark = pytest.mark.gpu
 
 
@@ -70,20 +72,16 @@ def test_conv1d_bits_do_not_depend_on_the_form(q, ctx, batch, ch, kern):
         np.testing.assert_array_equal(after[:, begin:end], ring[:, begin:end])
 
 
-@pytest.mark.parametrize("vocab,k", [(64, 64), (264, 1), (264, 64), (8192, 20), (8192, 64)])
-@pytest.mark.parametrize("ties", [False, True])
-def test_candidates_against_sort(q, ctx, vocab, k, ties):
-    """The candidate list equals a descending sort of the raw logits (lower
-    token first among equals): few tokens per slice, all logits equal (a zero
-    hidden row), penalized tokens, k up to 64."""
+def _candidate_model(q, ctx, vocab):
     from tests.model_util import build_small_model, small_dims, upload_model
     d, sched = small_dims()
     d["vocab"] = vocab
     model = upload_model(q, ctx, d, sched, build_small_model(d, sched, seed=vocab))
-    rt = q.Runtime(model, max_slots=1, max_batch=1, max_context=64, page_tokens=16, use_graphs=False)
-    prompt = np.arange(0, vocab, 3, dtype=np.int32)[:40]
-    slot = rt.slot_alloc(prompt)
-    rng = np.random.default_rng(k)
+    return d, model, q.Runtime(model, max_slots=1, max_batch=1, max_context=64, page_tokens=16, use_graphs=False)
+
+
+def _check_candidates(rt, d, slot, k, ties, rng):
+    vocab = d["vocab"]
     hidden = np.zeros(d["hidden"], np.float32) if ties else rng.standard_normal(d["hidden"]).astype(np.float32)
     print(f"candidates vocab {vocab} k {k} ties {ties}", flush=True)
     cand, raw = rt.head_candidates(slot, hidden, k, 1.25, penalty=1.3, raw_logits=True)
@@ -97,6 +95,36 @@ def test_candidates_against_sort(q, ctx, vocab, k, ties):
     np.testing.assert_array_equal(cand["token"][:k], order)
     np.testing.assert_array_equal(cand["value"][:k].view(np.uint32), v[order].view(np.uint32))
     assert np.all(cand["token"][k:] == -1) and np.all(np.isneginf(cand["value"][k:]))
+    return raw, order
+
+
+@pytest.mark.parametrize("vocab,k", [(64, 64), (264, 1), (264, 64), (8192, 20), (8192, 64)])
+@pytest.mark.parametrize("ties", [False, True])
+def test_candidates_against_sort(q, ctx, vocab, k, ties):
+    """The candidate list equals a descending sort of the raw logits (lower
+    token first among equals): few tokens per slice, all logits equal (a zero
+    hidden row), penalized tokens, k up to 64."""
+    d, model, rt = _candidate_model(q, ctx, vocab)
+    slot = rt.slot_alloc(np.arange(0, vocab, 3, dtype=np.int32)[:40])
+    _check_candidates(rt, d, slot, k, ties, np.random.default_rng(k))
+    rt.close()
+    model.close()
+
+
+@pytest.mark.parametrize("vocab", [20008, 248320])
+def test_candidates_of_many_tokens_per_slice(q, ctx, vocab):
+    """The same where a thread of a slice holds several tokens: 313 a slice
+    with a ragged last one, and the 3880 of the models' vocabulary (all 16 a
+    thread takes); every third token counted, so that penalties fall on every
+    place of a slice and move some of the best."""
+    d, model, rt = _candidate_model(q, ctx, vocab)
+    slot = rt.slot_alloc(np.arange(0, vocab, 3, dtype=np.int32))
+    rng = np.random.default_rng(vocab)
+    for k in (1, 20, 64):
+        _check_candidates(rt, d, slot, k, True, rng)
+        raw, order = _check_candidates(rt, d, slot, k, False, rng)
+        if k == 64:
+            assert set(order) != set(np.argsort(-raw)[:k])  # some of the best raw logits were counted
     rt.close()
     model.close()
 
@@ -151,13 +179,6 @@ def test_direct_gemm_forms(q, ctx, orc, rows, blocks, tokens):
     np.testing.assert_array_equal(few.view(np.uint32), got[:5].view(np.uint32))
 
 
-class _At:
-    """A place within a device array, as an operator's buffer argument."""
-
-    def __init__(self, array, offset):
-        self.array, self.ptr = array, type(array.ptr)(array.ptr.value + offset)
-
-
 @pytest.mark.parametrize("offset", [0, 160, 1024])
 @pytest.mark.parametrize("rows,blocks,tokens,x1", [(40, 9, 8, False), (40, 9, 7, True), (72, 3, 64, False),
                                                    (24, 17, 68, False), (24, 2, 67, True)])
@@ -184,7 +205,7 @@ def test_outputs_over_activations(q, ctx, orc, rows, blocks, tokens, x1, offset)
             host = np.zeros(offset + max(act.size, out_bytes), np.uint8)
             host[a_at:a_at + act.size] = act
             both = ctx.array(host)
-            f(ctx, dm, _At(both, a_at), _At(both, o_at), rows, tokens, blocks, stride)
+            f(ctx, dm, At(both, a_at), At(both, o_at), rows, tokens, blocks, stride)
             got = both.download()[o_at:o_at + out_bytes].view(np.float32).reshape(tokens, stride)[:, :rows]
             np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
 
