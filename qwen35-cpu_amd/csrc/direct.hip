@@ -15,10 +15,12 @@
 // lane needs one activation scale, which sits beside its codes in either
 // layout, and its four row scales are eight contiguous bytes of a tile.
 //
-// These launches are bound by latency; a chunk of KS blocks is loaded at a
-// time, as far ahead as the compiler schedules it. Per call,
-// against layout + split GEMM + reduce: 3584 x 1024, 16 vectors 11.6 -> 3.7 us;
-// 8224 x 1024, 7 vectors 11.6 -> 6.2 us; 4096 x 2560, 64 vectors 18.1 -> 8.2 us.
+// These launches are bound by latency. KS blocks are unrolled together; how
+// many of their loads are in flight is the compiler's choice (one tile keeps
+// within 42 registers, about half a chunk of eight), and forcing all of them
+// cost more in occupancy than it gave. Per call, against layout + split GEMM +
+// reduce: 3584 x 1024, 16 vectors 11.6 -> 4.2 us; 8224 x 1024, 7 vectors 11.6 ->
+// 6.2 us; 4096 x 2560, 64 vectors 18.7 -> 8.1 us.
 #include <algorithm>
 
 #include "q35_device.h"

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kPrepThreads) void prep_kernel(PrepArgs a) {
 // 128-column block), 16 lanes per token, so that it writes the four X4 blocks
 // -- 608 contiguous bytes -- whole. What bounds it is memory: with a token per
 // half wavefront the 32-byte pieces of a block came from four workgroups, and
-// 2048 x 9216 took 26.3-29.9 us (3.3-3.7 TB/s); this form 19.6 us (5.0 TB/s).
+// 2048 x 9216 took 28.8 us a call (3.4 TB/s); this form 21.2 us (4.6 TB/s).
 __global__ __launch_bounds__(kPrepThreads) void prep_x4_kernel(PrepArgs a) {
   const int K = a.K, nblk = K >> 7, lane = threadIdx.x & 63;
   const int groups = (a.tokens >> 2) * nblk;

@@ -22,7 +22,7 @@
 // (ballots and one barrier a round, about 20 rounds). What bounds it is that
 // chain of rounds, not the logits. Sorting every slice of 4096 keys in LDS
 // instead (78 barriers of 1024 threads) took 115 us for 16 rows of 248,320
-// logits and the second sort 37 us; this form 21 us and 12 us.
+// logits and the second sort 37 us; this form 20 us and 11 us.
 #include "q35_device.h"
 #include "q35_internal.h"
 
